@@ -228,12 +228,14 @@ hipError_t pair_energy(const float *xyz, int64_t n, const int64_t *offsets,
 {
   const float phic = shifted_phi_cutoff(cutoff);
   const int64_t nb = energy_blocks(n);
-  double *partials = (double *)dalloc(nb * sizeof(double), s);
+  // from the pool itself: the call returns while the kernels run, and it
+  // may be captured
+  double *partials = (double *)pool_alloc(nb * sizeof(double), s);
   if (!partials)
     return hipErrorOutOfMemory;
   const hipError_t e =
       launch_energy(xyz, n, offsets, indices, phic, order, partials, nb, energy, grad, s, true);
-  dfree(partials, s);
+  pool_free(partials, s);
   return e;
 }
 

@@ -26,7 +26,10 @@ void set_error(const std::string &msg);
     }                                                                          \
   } while (0)
 
-// Stream-ordered device allocation (hipMallocAsync on `stream`).
+// Stream-ordered device allocation: pool_* is hipMallocAsync on `stream`;
+// dalloc/dfree keep freed blocks per (device, stream) for the next call.
+void *pool_alloc(size_t bytes, hipStream_t stream);
+void pool_free(void *p, hipStream_t stream);
 void *dalloc(size_t bytes, hipStream_t stream);
 void dfree(void *p, hipStream_t stream);
 
