@@ -664,27 +664,83 @@ __global__ __launch_bounds__(256) void k_lin_q16(const INode *__restrict__ inode
   }
 }
 
+// Min / max over the wavefront, the bounds in lane 0.
+AXB_D void wave_bounds(float (&lo)[3], float (&hi)[3])
+{
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1)
+#pragma unroll
+    for (int d = 0; d < 3; ++d)
+    {
+      lo[d] = kmin(lo[d], __shfl_xor(lo[d], o, 64));
+      hi[d] = kmax(hi[d], __shfl_xor(hi[d], o, 64));
+    }
+}
+
+// Leaf records to their slots; points: a wavefront's 64 leaves are a block
+// of the leaf blocks, whose box it writes on the way.
 template <int G, int SI>
 __global__ __launch_bounds__(256) void k_lin_leaves(const float4 *__restrict__ leafrec,
                                                     int n,
                                                     const int32_t *__restrict__ C,
                                                     uint4 *__restrict__ slots, uint32_t total,
-                                                    uint32_t *err)
+                                                    float4 *__restrict__ blk, uint32_t *err)
 {
   constexpr uint32_t SL = leaf_slots<G>();
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n)
-    return;
-  const uint32_t pos = SL * (uint32_t)i + (uint32_t)SI * (uint32_t)C[i];
-  if (pos + SL > total)
-  {
-    raise_error(err, KERR_LAYOUT);
-    return;
-  }
   const uint4 *src = (const uint4 *)leafrec;
-  slots[pos] = src[SL * i];
-  if (SL == 2)
-    slots[pos + 1] = src[SL * i + 1];
+  uint4 rec = make_uint4(0u, 0u, 0u, 0u);
+  if (i < n)
+  {
+    rec = src[SL * i];
+    const uint32_t pos = SL * (uint32_t)i + (uint32_t)SI * (uint32_t)C[i];
+    if (pos + SL > total)
+      raise_error(err, KERR_LAYOUT);
+    else
+    {
+      slots[pos] = rec;
+      if (SL == 2)
+        slots[pos + 1] = src[SL * i + 1];
+    }
+  }
+  if constexpr (G == GEOM_POINTS)
+  {
+    const float c[3] = {bits_f(rec.x), bits_f(rec.y), bits_f(rec.z)};
+    float lo[3], hi[3];
+#pragma unroll
+    for (int d = 0; d < 3; ++d)
+    {
+      // kmin / kmax leave out a NaN coordinate in their second argument
+      lo[d] = i < n ? kmin(FLT_MAX, c[d]) : FLT_MAX;
+      hi[d] = i < n ? kmax(-FLT_MAX, c[d]) : -FLT_MAX;
+    }
+    wave_bounds(lo, hi);
+    if ((threadIdx.x & 63) == 0 && i < n)
+    {
+      blk[2 * (i / BLOCK_LEAVES)] = make_float4(lo[0], lo[1], lo[2], hi[0]);
+      blk[2 * (i / BLOCK_LEAVES) + 1] = make_float4(hi[1], hi[2], 0.f, 0.f);
+    }
+  }
+}
+
+// Boxes over 64 boxes of the level below (m of them, at `below`), one
+// wavefront each.
+__global__ __launch_bounds__(256) void k_block_boxes(const float4 *__restrict__ below,
+                                                     uint32_t m, float4 *__restrict__ out)
+{
+  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+  float lo[3] = {FLT_MAX, FLT_MAX, FLT_MAX}, hi[3] = {-FLT_MAX, -FLT_MAX, -FLT_MAX};
+  if (i < m)
+  {
+    const float4 a = below[2 * (size_t)i], b = below[2 * (size_t)i + 1];
+    lo[0] = a.x, lo[1] = a.y, lo[2] = a.z, hi[0] = a.w, hi[1] = b.x, hi[2] = b.y;
+  }
+  wave_bounds(lo, hi);
+  if ((threadIdx.x & 63) == 0 && i < m)
+  {
+    out[2 * (size_t)(i / 64)] = make_float4(lo[0], lo[1], lo[2], hi[0]);
+    out[2 * (size_t)(i / 64) + 1] = make_float4(hi[1], hi[2], 0.f, 0.f);
+  }
 }
 
 template <int G>
@@ -845,6 +901,14 @@ hipError_t build_tree(const float *values, int64_t n, int geometry,
   int32_t *spine_count = (int32_t *)dalloc(nlists * sizeof(int32_t), stream);
   int32_t *spine_list = (int32_t *)dalloc(nlists * CLIMB_LEAVES * sizeof(int32_t), stream);
   out.C = (int32_t *)dalloc(n * sizeof(int32_t), stream);
+  const BlockLevels bl = block_levels(n);
+  if (geometry == GEOM_POINTS)
+  {
+    out.leaves = (uint4 *)leafrec; // kept with the tree
+    out.blk = (float4 *)dalloc(2 * (size_t)bl.boxes * sizeof(float4), stream);
+    if (!out.blk)
+      return hipErrorOutOfMemory;
+  }
   int32_t *leaf_rope = keep_topology ? (int32_t *)dalloc(n * sizeof(int32_t), stream) : nullptr;
   if (!keys0 || !keys1 || !vals0 || !vals1 || !hist || !partials || !ws || !ranges ||
       !inodes || !leafrec || !c || !top || !pending || !spine_count ||
@@ -931,14 +995,14 @@ hipError_t build_tree(const float *values, int64_t n, int geometry,
         AXB_LAUNCH(k_lin_fp32<GEOM_POINTS>, dim3(gi), dim3(256), 0, stream, inodes,
                            nint, out.C, out.slots, (uint32_t)out.max_slots, err);
         AXB_LAUNCH((k_lin_leaves<GEOM_POINTS, 2>), dim3(gl), dim3(256), 0, stream,
-                           leafrec, ni, out.C, out.slots, (uint32_t)out.max_slots, err);
+                           leafrec, ni, out.C, out.slots, (uint32_t)out.max_slots, out.blk, err);
       }
       else
       {
         AXB_LAUNCH(k_lin_fp32<GEOM_BOXES>, dim3(gi), dim3(256), 0, stream, inodes,
                            nint, out.C, out.slots, (uint32_t)out.max_slots, err);
         AXB_LAUNCH((k_lin_leaves<GEOM_BOXES, 2>), dim3(gl), dim3(256), 0, stream,
-                           leafrec, ni, out.C, out.slots, (uint32_t)out.max_slots, err);
+                           leafrec, ni, out.C, out.slots, (uint32_t)out.max_slots, out.blk, err);
       }
     }
     else
@@ -949,7 +1013,7 @@ hipError_t build_tree(const float *values, int64_t n, int geometry,
                    inodes, ni, spine_count, spine_list, (int)nlists, top, out.C, out.scene,
                    out.slots, (uint32_t)out.max_slots, err);
         AXB_LAUNCH((k_lin_leaves<GEOM_POINTS, 1>), dim3(gl), dim3(256), 0, stream,
-                           leafrec, ni, out.C, out.slots, (uint32_t)out.max_slots, err);
+                           leafrec, ni, out.C, out.slots, (uint32_t)out.max_slots, out.blk, err);
       }
       else
       {
@@ -957,12 +1021,16 @@ hipError_t build_tree(const float *values, int64_t n, int geometry,
                    inodes, ni, spine_count, spine_list, (int)nlists, top, out.C, out.scene,
                    out.slots, (uint32_t)out.max_slots, err);
         AXB_LAUNCH((k_lin_leaves<GEOM_BOXES, 1>), dim3(gl), dim3(256), 0, stream,
-                           leafrec, ni, out.C, out.slots, (uint32_t)out.max_slots, err);
+                           leafrec, ni, out.C, out.slots, (uint32_t)out.max_slots, out.blk, err);
       }
     }
   }
   if (geometry == GEOM_POINTS)
   {
+    for (uint32_t l = 1; l < bl.levels; ++l)
+      AXB_LAUNCH(k_block_boxes, dim3(grid_for(bl.count[l - 1])), dim3(256), 0, stream,
+                 out.blk + 2 * (size_t)bl.at[l - 1], bl.count[l - 1],
+                 out.blk + 2 * (size_t)bl.at[l]);
     if (node_format == NODES_FP32)
       AXB_LAUNCH((k_pad_tail<1, 2>), dim3(1), dim3(64), 0, stream, out.slots, out.C, ni);
     else
@@ -983,7 +1051,8 @@ hipError_t build_tree(const float *values, int64_t n, int geometry,
   dfree(partials, stream);
   dfree(ws, stream);
   dfree(ranges, stream);
-  dfree(leafrec, stream);
+  if (geometry != GEOM_POINTS)
+    dfree(leafrec, stream);
   dfree(c, stream);
   dfree(top, stream);
   dfree(pending, stream);

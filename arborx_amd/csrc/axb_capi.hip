@@ -527,6 +527,12 @@ static TreeView view_of(const axb_bvh *t, uint32_t *err)
   tv.C = t->b.C;
   tv.err = err;
   tv.visits = visit_counters();
+  tv.leaves = t->b.leaves;
+  tv.blk = t->b.blk;
+  const BlockLevels bl = block_levels(t->n);
+  tv.blk_levels = (int32_t)bl.levels;
+  for (int l = 0; l < BLOCK_LEVELS_MAX; ++l)
+    tv.blk_at[l] = bl.at[l], tv.blk_count[l] = bl.count[l];
   for (int d = 0; d < 3; ++d)
   {
     tv.scene.lo[d] = t->bounds[d];
@@ -698,6 +704,8 @@ void axb_bvh_destroy(axb_bvh *t)
   dfree(t->b.slots, s);
   dfree(t->b.scene, s);
   dfree(t->b.C, s);
+  dfree(t->b.leaves, s);
+  dfree(t->b.blk, s);
   dfree(t->b.keys, s);
   dfree(t->b.perm, s);
   dfree(t->b.leaf_rope, s);
@@ -742,15 +750,15 @@ axb_status axb_bvh_export_topology(const axb_bvh *t, uint64_t *keys, uint32_t *p
   return AXB_OK;
 }
 
-// Morton-32 processing order of predicates (CrsGraphWrapperImpl.hpp:407-419).
-// exact: the permutation that sorts the centroids by their 30-bit Morton
-// codes (ties by position); otherwise by the top 24 bits of the codes (8 per
-// axis, cells of 1/256 of the scene per axis), one radix pass fewer -- the
-// processing order of a query batch only decides which predicates share a
-// wavefront, never a result.
-static axb_status morton_order(const float *scene, uint32_t *d_err, int pred_kind,
+// Processing order of predicates (CrsGraphWrapperImpl.hpp:407-419) along a
+// curve through the cells of the scene.  CURVE_MORTON30: the permutation
+// that sorts the centroids by their 30-bit Morton codes (ties by position);
+// the 24-bit curves (cells of 1/256 of the scene per axis) take one radix
+// pass fewer -- the processing order of a query batch only decides which
+// predicates share a wavefront, never a result.
+static axb_status curve_order(const float *scene, uint32_t *d_err, int pred_kind,
                                const float *preds, int64_t nq, hipStream_t s,
-                               uint32_t **order_out, void **to_free, bool exact = false)
+                               uint32_t **order_out, void **to_free, int curve)
 {
   *order_out = nullptr;
   if (nq < 2)
@@ -758,7 +766,7 @@ static axb_status morton_order(const float *scene, uint32_t *d_err, int pred_kin
   // the sort's look-back words carry 30-bit counts
   if (nq >= MAX_SORTED_PREDICATES)
     AXB_FAIL(AXB_ERR_INVALID_ARGUMENT, "query: sort_predicates needs fewer than 2^30 predicates");
-  const int passes = exact ? 4 : 3;
+  const int passes = curve == CURVE_MORTON30 ? 4 : 3;
   const size_t ws_bytes = sort_workspace_bytes(nq, 4, 4);
   // one block: keys0 keys1 vals0 vals1 hist workspace
   const size_t a = (size_t)nq * 4;
@@ -772,7 +780,7 @@ static axb_status morton_order(const float *scene, uint32_t *d_err, int pred_kin
   uint32_t *hist = (uint32_t *)(blk + off_h);
   hipError_t e = fill_u32(hist, 0u, 4 * 256, s);
   if (e == hipSuccess)
-    e = launch_pred_morton32(pred_kind, preds, nq, scene, exact ? 0 : 6, k0, hist, s);
+    e = launch_pred_keys(pred_kind, preds, nq, scene, curve, k0, hist, s);
   if (e == hipSuccess)
     e = radix_sort_pairs_u32(k0, k1, v0, v1, nq, passes, hist, blk + off_ws, d_err, s);
   if (e != hipSuccess)
@@ -788,9 +796,9 @@ static axb_status morton_order(const float *scene, uint32_t *d_err, int pred_kin
 
 static axb_status predicate_order(const axb_bvh *t, uint32_t *err, int pred_kind,
                                   const float *preds, int64_t nq, hipStream_t s,
-                                  uint32_t **order_out, void **to_free, bool exact = false)
+                                  uint32_t **order_out, void **to_free, int curve)
 {
-  return morton_order(t->b.scene, err, pred_kind, preds, nq, s, order_out, to_free, exact);
+  return curve_order(t->b.scene, err, pred_kind, preds, nq, s, order_out, to_free, curve);
 }
 
 } // extern "C"
@@ -1045,7 +1053,7 @@ static axb_status query_spatial(const axb_bvh *t, int pred_kind, const float *pr
     Region perm_region(ordered ? "ArborX::BVH::query::ordered_spatial::compute_permutation"
                                : "ArborX::BVH::query::spatial::compute_permutation");
     axb_status st = predicate_order(t, err.p, ordered ? PRED_RAYS : pred_kind, preds, nq, s,
-                                    &order, &order_blk);
+                                    &order, &order_blk, CURVE_HILBERT24);
     if (st != AXB_OK)
       return st;
   }
@@ -1287,7 +1295,7 @@ axb_status axb_bvh_predicate_order(const axb_bvh *t, int32_t predicate_kind,
     AXB_FAIL(AXB_ERR_OUT_OF_MEMORY, "axb_bvh_predicate_order: out of device memory");
   uint32_t *ord = nullptr;
   void *blk = nullptr;
-  axb_status st = predicate_order(t, err.p, predicate_kind, preds, nq, s, &ord, &blk, true);
+  axb_status st = predicate_order(t, err.p, predicate_kind, preds, nq, s, &ord, &blk, CURVE_MORTON30);
   if (st != AXB_OK)
     return st;
   hipError_t e = hipMemcpyAsync(order, ord, (size_t)nq * sizeof(uint32_t),
@@ -1354,21 +1362,35 @@ axb_status axb_bvh_neighbor_list(const axb_bvh *t, float radius, int32_t full,
   if (!rowof)
     AXB_FAIL(AXB_ERR_OUT_OF_MEMORY, "axb_bvh_neighbor_list: out of device memory");
   const bool f = full != 0;
-  // lanes walk the leaves in tree order (already Morton-sorted)
+  // Full lists: leaves in Hilbert order, 64 lanes searching together; half
+  // lists walk the leaves in tree order.
+  uint32_t *order = nullptr;
+  void *order_blk = nullptr;
+  if (f)
+  {
+    axb_status st = predicate_order(t, err.p, PRED_LEAVES, (const float *)t->b.leaves, n, s,
+                                    &order, &order_blk, CURVE_HILBERT24);
+    if (st != AXB_OK)
+    {
+      dfree(rowof, s);
+      return st;
+    }
+  }
   auto first = [&](int mode, int32_t *out, int32_t B) {
-    return launch_nlist(tv, t->node_format, f, radius, n, nullptr, offsets, out, B, rowof, mode,
+    return launch_nlist(tv, t->node_format, f, radius, n, order, offsets, out, B, rowof, mode, f,
                         s);
   };
   // the overflow list holds leaf positions
   auto fill = [&](const uint32_t *list, int64_t n_list, int32_t *out) {
-    return launch_nlist(tv, t->node_format, f, radius, n_list, list, offsets, out, 0, nullptr,
-                        MODE_FILL, s);
+    return launch_nlist(tv, t->node_format, f, radius, n_list, list ? list : order, offsets, out,
+                        0, nullptr, MODE_FILL, f, s);
   };
   // rows of 96, as for queries: the 2M-atom FCC lattice's ~83 neighbours
   // per row take 5.1 ms with rows of 64 (most rows walked twice), 2.4 ms
   // with 96; ~32 uniform neighbours 6.2 vs 6.3 ms at 10M points
   axb_status st = crs_query(err.p, n, policy, rowof, true, first, fill, offsets, indices,
                             nnz_host, s, "axb_bvh_neighbor_list", nullptr, 96);
+  dfree(order_blk, s);
   dfree(rowof, s);
   return st;
 }
@@ -1502,7 +1524,8 @@ axb_status axb_bvh_query_nearest(const axb_bvh *t, const float *points, int64_t 
     if (e == hipSuccess && policy.sort_predicates)
     {
       Region perm_region("ArborX::BVH::query::nearest::compute_permutation");
-      axb_status st = predicate_order(t, err.p, PRED_RADIUS, points, nq, s, &order, &order_blk);
+      axb_status st = predicate_order(t, err.p, PRED_RADIUS, points, nq, s, &order, &order_blk,
+                                      CURVE_MORTON24);
       if (st != AXB_OK)
       {
         out_free(*indices, s);
@@ -1652,7 +1675,8 @@ axb_status axb_pair_energy(const float *xyz, int64_t n, const int64_t *offsets,
     if (e == hipSuccess)
       e = scene_box(xyz, n, AXB_GEOMETRY_POINTS, scene, s);
     if (e == hipSuccess &&
-        morton_order(scene, d_err, PRED_RADIUS, xyz, n, s, &order, &order_blk) != AXB_OK)
+        curve_order(scene, d_err, PRED_RADIUS, xyz, n, s, &order, &order_blk, CURVE_MORTON24) !=
+            AXB_OK)
       e = hipErrorOutOfMemory;
   }
   if (e == hipSuccess)

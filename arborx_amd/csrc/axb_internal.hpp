@@ -183,12 +183,41 @@ struct BuildOut
   int64_t total_slots; // records actually stored (SL * n + SI * C[n - 1])
   float *scene;        // 6 floats (device)
   int32_t *C;          // n: inclusive prefix of left-spine counts
+  uint4 *leaves;       // point trees of n >= 2: the leaf records in leaf order
+  float4 *blk;         // and the boxes over 64 of them, 64 of those, ... (BlockLevels)
   // reference-form topology (kept on request)
   uint64_t *keys;
   uint32_t *perm;
   int32_t *leaf_rope;
   INode *inodes;
 };
+
+// Implicit 64-wide tree over the sorted leaves of a point tree: box i of
+// level 0 bounds leaves [64 i, 64 i + 64), box i of level l boxes [64 i, 64 i
+// + 64) of level l - 1; the top level has at most 64.  A box is two float4
+// {lo.x lo.y lo.z hi.x}{hi.y hi.z 0 0}; level l starts at box at[l].
+constexpr int BLOCK_LEAVES = 64;
+constexpr int BLOCK_LEVELS_MAX = 4; // 2^30 leaves
+struct BlockLevels
+{
+  uint32_t levels, boxes;
+  uint32_t at[BLOCK_LEVELS_MAX], count[BLOCK_LEVELS_MAX];
+};
+inline BlockLevels block_levels(int64_t n)
+{
+  BlockLevels b{};
+  int64_t c = div_up(n > 0 ? n : 1, BLOCK_LEAVES);
+  while (true)
+  {
+    b.at[b.levels] = b.boxes;
+    b.count[b.levels] = (uint32_t)c;
+    b.boxes += (uint32_t)c;
+    ++b.levels;
+    if (c <= 64 || b.levels == BLOCK_LEVELS_MAX)
+      return b;
+    c = div_up(c, 64);
+  }
+}
 
 struct TreeView
 {
@@ -200,6 +229,10 @@ struct TreeView
   float ss[3];   // Q16 scale of the scene frame
   uint32_t *err; // kernel error word
   unsigned long long *visits; // optional visit counters (see visit_counters)
+  const uint4 *leaves;        // point trees of n >= 2 (else null), with the
+  const float4 *blk;          // boxes of BlockLevels
+  int32_t blk_levels;
+  uint32_t blk_at[BLOCK_LEVELS_MAX], blk_count[BLOCK_LEVELS_MAX];
 };
 
 constexpr int MODE_COUNT = 0;
@@ -399,21 +432,26 @@ struct KnnScratch
 };
 int knn_row_capacity(int k, int n);
 hipError_t launch_knn_offsets(int64_t *offsets, int64_t nq, int64_t per, hipStream_t s);
-// keys = the predicates' 30-bit Morton codes >> shift, and the histograms of
-// their four 8-bit digits
-hipError_t launch_pred_morton32(int pred_kind, const float *preds, int64_t nq,
-                                const float *scene, int shift, uint32_t *keys, uint32_t *hist,
-                                hipStream_t s);
+// keys = the predicates' 30-bit Morton codes, their top 24 bits, or 24-bit
+// indices along the Hilbert curve, and the histograms of their 8-bit digits
+// (pred_kind PRED_LEAVES: a tree's leaf records, 4 floats apart).
+constexpr int PRED_LEAVES = 16;
+constexpr int CURVE_MORTON30 = 0;
+constexpr int CURVE_MORTON24 = 1;
+constexpr int CURVE_HILBERT24 = 2;
+hipError_t launch_pred_keys(int pred_kind, const float *preds, int64_t nq, const float *scene,
+                            int curve, uint32_t *keys, uint32_t *hist, hipStream_t s);
 hipError_t launch_compact(const int32_t *buf, int64_t nq, int32_t buffer,
                           const int64_t *offsets, int32_t *out, hipStream_t s);
 hipError_t launch_overflow_list(const uint8_t *over_flags, const uint32_t *order, int64_t nq,
                                 bool emit_index, uint32_t *ovf, uint32_t *ovf_n, hipStream_t s);
 // Neighbour list of a point tree: lane t takes leaf position list[t] (t when
-// list is nullptr); rows are the leaves' values.  rowof (leaf position ->
+// list is nullptr); rows are the leaves' values.  group: 64 lanes search
+// together (full lists; the positions are sorted along a curve).  rowof (leaf position ->
 // row) is written when non-null.
 hipError_t launch_nlist(const TreeView &tv, int node_format, bool full, float radius, int64_t nl,
                         const uint32_t *list, int64_t *offsets, int32_t *out, int32_t buffer,
-                        uint32_t *rowof, int mode, hipStream_t s);
+                        uint32_t *rowof, int mode, bool group, hipStream_t s);
 // Half -> full neighbour list: counts into cnt (zeroed, n + 1 entries), then
 // after the scan into out_offsets, the fill (cursor: n scratch entries).
 hipError_t launch_h2f_count(const int64_t *offsets, const int32_t *indices, int64_t n,

@@ -24,6 +24,7 @@
 // LDS candidate buffer); k > 64 uses a binary max-heap in the output row
 // (the reference's NearestBufferProvider scheme, NearestBufferProvider.hpp:
 // 23-73).
+#include "axb_group.hpp"
 #include "axb_internal.hpp"
 
 #include <algorithm>
@@ -77,6 +78,45 @@ __global__ __launch_bounds__(256) void k_spatial(
     rope_walk<F, G, PK, SLOTS>(tv, pr, 0u, tv.total, ~0u, rw, v_int, v_leaf);
     row_epilogue(tv, rw, offsets, q, COUNT ? v_int : 0u, COUNT ? v_leaf : 0u);
   }
+}
+
+// Spheres against points, 64 lanes searching together (axb_group.hpp).
+template <int F, int PK, int MODE, bool COUNT>
+__global__ __launch_bounds__(256, 6) void k_spatial_group(
+    TreeView tv, const float *__restrict__ preds, int64_t nq, float radius,
+    const uint32_t *__restrict__ order, int64_t *__restrict__ offsets,
+    int32_t *__restrict__ out, int32_t buffer)
+{
+  __shared__ GroupLds s_group[4];
+  const int64_t t = (int64_t)xcd_block(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
+  // lanes past the last predicate take part in the wavefront's search
+  const bool real = t < nq;
+  int64_t q = 0;
+  float x = 0.f, y = 0.f, z = 0.f, r = -1.f;
+  if (real)
+  {
+    q = order ? (int64_t)order[t] : t;
+    const float *p = preds + (PK == PRED_SPHERES ? 4 : 3) * q;
+    x = p[0], y = p[1], z = p[2];
+    r = PK == PRED_SPHERES ? p[3] : radius;
+  }
+  const float thr = sqrt_threshold(r);
+  const bool active = real && r >= 0.f && fabsf(x) < INFINITY && fabsf(y) < INFINITY &&
+                      fabsf(z) < INFINITY;
+  RowWriter<MODE> rw;
+  if (real)
+    rw.init(out, offsets, q, buffer);
+  uint32_t v_int = 0, v_leaf = 0;
+  if (!group_walk<false>(tv, s_group[threadIdx.x >> 6], x, y, z, r, thr, active, -1, rw, v_int, v_leaf))
+  {
+    if (real)
+    {
+      const SpatialPred pr = sphere_pred(x, y, z, r);
+      rope_walk<F, GEOM_POINTS, PK>(tv, pr, 0u, tv.total, ~0u, rw, v_int, v_leaf);
+    }
+  }
+  if (real)
+    row_epilogue(tv, rw, offsets, q, COUNT ? v_int : 0u, COUNT ? v_leaf : 0u);
 }
 
 // Rows of leaf slots hit by each ray -> rows of values in (distance, index)
@@ -267,6 +307,53 @@ __global__ __launch_bounds__(256) void k_nlist(TreeView tv, float radius, int64_
   rope_walk<F, GEOM_POINTS, PRED_SPHERES>(tv, pr, 0u, FULL ? tv.total : self, self, rw, v_int,
                                           v_leaf);
   row_epilogue(tv, rw, offsets, q, v_int, v_leaf);
+}
+
+// Full neighbour lists, 64 lanes searching together: lane t takes the leaf
+// at position order[t] (the leaves sorted along the Hilbert curve, or a list
+// of positions) and the sphere {its point, radius}.
+template <int F, int MODE>
+__global__ __launch_bounds__(256, 6) void k_nlist_group(TreeView tv, float radius, int64_t nl,
+                                                        const uint32_t *__restrict__ order,
+                                                        int64_t *__restrict__ offsets,
+                                                        int32_t *__restrict__ out,
+                                                        int32_t buffer,
+                                                        uint32_t *__restrict__ rowof)
+{
+  __shared__ GroupLds s_group[4];
+  const int64_t t = (int64_t)xcd_block(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
+  const bool real = t < nl;
+  int64_t q = 0;
+  uint32_t L = 0;
+  float x = 0.f, y = 0.f, z = 0.f;
+  RowWriter<MODE> rw;
+  if (real)
+  {
+    L = order ? order[t] : (uint32_t)t;
+    const uint4 s = tv.leaves[L];
+    x = bits_f(s.x), y = bits_f(s.y), z = bits_f(s.z);
+    q = ~(int32_t)s.w;
+    if (rowof)
+      rowof[L] = (uint32_t)q;
+    rw.init(out, offsets, q, buffer);
+  }
+  const float thr = sqrt_threshold(radius);
+  const bool active =
+      real && fabsf(x) < INFINITY && fabsf(y) < INFINITY && fabsf(z) < INFINITY;
+  uint32_t v_int = 0, v_leaf = 0;
+  if (!group_walk<true>(tv, s_group[threadIdx.x >> 6], x, y, z, radius, thr, active, (int32_t)q,
+                        rw, v_int, v_leaf))
+  {
+    if (real)
+    {
+      constexpr uint32_t SL = leaf_slots<GEOM_POINTS>(), SI = internal_slots<F>();
+      const uint32_t self = SL * L + SI * (uint32_t)tv.C[L];
+      const SpatialPred pr = sphere_pred(x, y, z, radius);
+      rope_walk<F, GEOM_POINTS, PRED_SPHERES>(tv, pr, 0u, tv.total, self, rw, v_int, v_leaf);
+    }
+  }
+  if (real)
+    row_epilogue(tv, rw, offsets, q, v_int, v_leaf);
 }
 
 // ------------------------------------------------------------ nearest
@@ -1109,12 +1196,49 @@ __global__ void k_knn_offsets(int64_t *offsets, int64_t nq, int64_t per)
     offsets[i] = i * per;
 }
 
-// Morton-32 code of predicate centroids in the tree's scene box
-// (SpaceFillingCurves.hpp:31-43, CrsGraphWrapperImpl.hpp:407-419) plus the
-// digit histograms of the 4 radix passes.
-template <int PK>
-__global__ __launch_bounds__(256) void k_pred_morton32(
-    const float *__restrict__ preds, int64_t nq, const float *__restrict__ scene, int shift,
+// Index of a cell of the 256^3 grid along the Hilbert curve (the transpose
+// form of J. Skilling, "Programming the Hilbert curve", AIP Conf. Proc. 707,
+// 2004: Gray decoding after undoing the rotations level by level).
+// Consecutive cells always share a face, so 64 consecutive predicates lie
+// close together; along the Morton curve a run of 64 of uniform points has
+// twice the leaves within reach of its box (900 against 490 at a radius of
+// ~32 neighbours).
+AXB_D uint32_t hilbert24(uint32_t x, uint32_t y, uint32_t z)
+{
+#pragma unroll
+  for (uint32_t q = 128u; q > 1u; q >>= 1)
+  {
+    const uint32_t p = q - 1u;
+    x ^= (x & q) ? p : 0u;
+    uint32_t t = (x ^ y) & p;
+    if (y & q)
+      x ^= p;
+    else
+      x ^= t, y ^= t;
+    t = (x ^ z) & p;
+    if (z & q)
+      x ^= p;
+    else
+      x ^= t, z ^= t;
+  }
+  y ^= x;
+  z ^= y;
+  uint32_t t = 0u;
+#pragma unroll
+  for (uint32_t q = 128u; q > 1u; q >>= 1)
+    t ^= (z & q) ? q - 1u : 0u;
+  x ^= t, y ^= t, z ^= t;
+  return (expand2_u32(x) << 2) | (expand2_u32(y) << 1) | expand2_u32(z);
+}
+
+// Keys of the processing order of a batch of predicates, from their
+// centroids in the tree's scene box, plus the digit histograms of the radix
+// passes: the Morton-32 code (SpaceFillingCurves.hpp:31-43,
+// CrsGraphWrapperImpl.hpp:407-419) or its top 24 bits, or 24 bits along the
+// Hilbert curve.
+template <int PK, int CURVE>
+__global__ __launch_bounds__(256) void k_pred_keys(
+    const float *__restrict__ preds, int64_t nq, const float *__restrict__ scene,
     uint32_t *__restrict__ keys, uint32_t *__restrict__ hist)
 {
   __shared__ uint32_t s_h[4 * 256];
@@ -1142,13 +1266,16 @@ __global__ __launch_bounds__(256) void k_pred_morton32(
       const float *v = preds + (PK == PRED_SPHERES ? 4 : 3) * i;
       cx = v[0], cy = v[1], cz = v[2];
     }
-    const uint32_t k = morton32(translate_and_scale(cx, a0, b0),
-                                translate_and_scale(cy, a1, b1),
-                                translate_and_scale(cz, a2, b2)) >>
-                       shift;
+    const float ux = translate_and_scale(cx, a0, b0), uy = translate_and_scale(cy, a1, b1),
+                uz = translate_and_scale(cz, a2, b2);
+    const uint32_t k = CURVE == CURVE_HILBERT24
+                           ? hilbert24((uint32_t)kclamp(ux * 256.f, 0.f, 255.f),
+                                       (uint32_t)kclamp(uy * 256.f, 0.f, 255.f),
+                                       (uint32_t)kclamp(uz * 256.f, 0.f, 255.f))
+                           : morton32(ux, uy, uz) >> (CURVE == CURVE_MORTON24 ? 6 : 0);
     keys[i] = k;
 #pragma unroll
-    for (int p = 0; p < 4; ++p)
+    for (int p = 0; p < (CURVE == CURVE_MORTON30 ? 4 : 3); ++p)
       atomicAdd(&s_h[p * 256 + ((k >> (8 * p)) & 255u)], 1u);
   }
   __syncthreads();
@@ -1328,12 +1455,56 @@ static hipError_t launch_spatial_fg(const TreeView &tv, const float *preds, int6
                                                           out, buffer, mode, s);
 }
 
+// Spheres against a point tree go to the group walk when the predicates are
+// not far fewer than the points (64 of them must lie close together).
+// Rows written again (MODE_FILL) come from such a batch and lie in its
+// densest parts.
+static bool group_rule(const TreeView &tv, int64_t nq, int mode)
+{
+  return tv.leaves && (mode == MODE_FILL || nq * 8 >= tv.n);
+}
+
+template <int F, int PK, bool COUNT>
+static hipError_t launch_group_c(const TreeView &tv, const float *preds, int64_t nq,
+                                 float radius, const uint32_t *order, int64_t *offsets,
+                                 int32_t *out, int32_t buffer, int mode, hipStream_t s)
+{
+  if (mode == MODE_COUNT)
+    AXB_LAUNCH((k_spatial_group<F, PK, MODE_COUNT, COUNT>), dim3(grid_of(nq)), dim3(256), 0, s,
+               tv, preds, nq, radius, order, offsets, out, buffer);
+  else if (mode == MODE_FILL)
+    AXB_LAUNCH((k_spatial_group<F, PK, MODE_FILL, COUNT>), dim3(grid_of(nq)), dim3(256), 0, s,
+               tv, preds, nq, radius, order, offsets, out, buffer);
+  else
+    AXB_LAUNCH((k_spatial_group<F, PK, MODE_BUFFER, COUNT>), dim3(grid_of(nq)), dim3(256), 0, s,
+               tv, preds, nq, radius, order, offsets, out, buffer);
+  return hipGetLastError();
+}
+template <int PK>
+static hipError_t launch_group(const TreeView &tv, int F, const float *preds, int64_t nq,
+                               float radius, const uint32_t *order, int64_t *offsets,
+                               int32_t *out, int32_t buffer, int mode, hipStream_t s)
+{
+  if (F == NODES_FP32)
+    return tv.visits ? launch_group_c<NODES_FP32, PK, true>(tv, preds, nq, radius, order,
+                                                            offsets, out, buffer, mode, s)
+                     : launch_group_c<NODES_FP32, PK, false>(tv, preds, nq, radius, order,
+                                                             offsets, out, buffer, mode, s);
+  return tv.visits ? launch_group_c<NODES_Q16, PK, true>(tv, preds, nq, radius, order, offsets,
+                                                         out, buffer, mode, s)
+                   : launch_group_c<NODES_Q16, PK, false>(tv, preds, nq, radius, order, offsets,
+                                                          out, buffer, mode, s);
+}
+
 template <int PK>
 static hipError_t launch_spatial_p(const TreeView &tv, int F, int G, const float *preds,
                                    int64_t nq, float radius, const uint32_t *order,
                                    int64_t *offsets, int32_t *out, int32_t buffer, int mode,
                                    hipStream_t s)
 {
+  if constexpr (PK != PRED_BOXES)
+    if (G == GEOM_POINTS && group_rule(tv, nq, mode))
+      return launch_group<PK>(tv, F, preds, nq, radius, order, offsets, out, buffer, mode, s);
   if (F == NODES_FP32 && G == GEOM_POINTS)
     return launch_spatial_fg<NODES_FP32, GEOM_POINTS, PK>(tv, preds, nq, radius, order, offsets,
                                                           out, buffer, mode, s);
@@ -1642,24 +1813,34 @@ hipError_t launch_knn_offsets(int64_t *offsets, int64_t nq, int64_t per, hipStre
   return hipGetLastError();
 }
 
-hipError_t launch_pred_morton32(int pred_kind, const float *preds, int64_t nq,
-                                const float *scene, int shift, uint32_t *keys, uint32_t *hist,
-                                hipStream_t s)
+template <int CURVE>
+static hipError_t launch_pred_keys_c(int pred_kind, const float *preds, int64_t nq,
+                                     const float *scene, uint32_t *keys, uint32_t *hist,
+                                     hipStream_t s)
 {
   const unsigned g = (unsigned)std::min<int64_t>(2048, div_up(nq, 256));
   if (pred_kind == PRED_RAYS)
-    AXB_LAUNCH(k_pred_morton32<PRED_RAYS>, dim3(g), dim3(256), 0, s, preds, nq, scene, shift, keys,
-               hist);
-  else if (pred_kind == PRED_SPHERES)
-    AXB_LAUNCH(k_pred_morton32<PRED_SPHERES>, dim3(g), dim3(256), 0, s, preds, nq,
-                       scene, shift, keys, hist);
+    AXB_LAUNCH((k_pred_keys<PRED_RAYS, CURVE>), dim3(g), dim3(256), 0, s, preds, nq, scene,
+               keys, hist);
+  else if (pred_kind == PRED_SPHERES || pred_kind == PRED_LEAVES)
+    AXB_LAUNCH((k_pred_keys<PRED_SPHERES, CURVE>), dim3(g), dim3(256), 0, s, preds, nq, scene,
+               keys, hist);
   else if (pred_kind == PRED_BOXES)
-    AXB_LAUNCH(k_pred_morton32<PRED_BOXES>, dim3(g), dim3(256), 0, s, preds, nq, scene,
-               shift, keys, hist);
+    AXB_LAUNCH((k_pred_keys<PRED_BOXES, CURVE>), dim3(g), dim3(256), 0, s, preds, nq, scene,
+               keys, hist);
   else
-    AXB_LAUNCH(k_pred_morton32<PRED_RADIUS>, dim3(g), dim3(256), 0, s, preds, nq,
-                       scene, shift, keys, hist);
+    AXB_LAUNCH((k_pred_keys<PRED_RADIUS, CURVE>), dim3(g), dim3(256), 0, s, preds, nq, scene,
+               keys, hist);
   return hipGetLastError();
+}
+hipError_t launch_pred_keys(int pred_kind, const float *preds, int64_t nq, const float *scene,
+                            int curve, uint32_t *keys, uint32_t *hist, hipStream_t s)
+{
+  if (curve == CURVE_HILBERT24)
+    return launch_pred_keys_c<CURVE_HILBERT24>(pred_kind, preds, nq, scene, keys, hist, s);
+  if (curve == CURVE_MORTON24)
+    return launch_pred_keys_c<CURVE_MORTON24>(pred_kind, preds, nq, scene, keys, hist, s);
+  return launch_pred_keys_c<CURVE_MORTON30>(pred_kind, preds, nq, scene, keys, hist, s);
 }
 
 hipError_t launch_compact(const int32_t *buf, int64_t nq, int32_t buffer,
@@ -1699,12 +1880,35 @@ static hipError_t launch_nlist_f(const TreeView &tv, float radius, int64_t nl,
   return hipGetLastError();
 }
 
+template <int F>
+static hipError_t launch_nlist_group(const TreeView &tv, float radius, int64_t nl,
+                                     const uint32_t *list, int64_t *offsets, int32_t *out,
+                                     int32_t buffer, uint32_t *rowof, int mode, hipStream_t s)
+{
+  if (mode == MODE_COUNT)
+    AXB_LAUNCH((k_nlist_group<F, MODE_COUNT>), dim3(grid_of(nl)), dim3(256), 0, s, tv, radius,
+               nl, list, offsets, out, buffer, rowof);
+  else if (mode == MODE_FILL)
+    AXB_LAUNCH((k_nlist_group<F, MODE_FILL>), dim3(grid_of(nl)), dim3(256), 0, s, tv, radius,
+               nl, list, offsets, out, buffer, rowof);
+  else
+    AXB_LAUNCH((k_nlist_group<F, MODE_BUFFER>), dim3(grid_of(nl)), dim3(256), 0, s, tv, radius,
+               nl, list, offsets, out, buffer, rowof);
+  return hipGetLastError();
+}
+
 hipError_t launch_nlist(const TreeView &tv, int node_format, bool full, float radius, int64_t nl,
                         const uint32_t *list, int64_t *offsets, int32_t *out, int32_t buffer,
-                        uint32_t *rowof, int mode, hipStream_t s)
+                        uint32_t *rowof, int mode, bool group, hipStream_t s)
 {
   if (nl <= 0)
     return hipSuccess;
+  if (group && full && tv.leaves)
+    return node_format == NODES_Q16
+               ? launch_nlist_group<NODES_Q16>(tv, radius, nl, list, offsets, out, buffer, rowof,
+                                               mode, s)
+               : launch_nlist_group<NODES_FP32>(tv, radius, nl, list, offsets, out, buffer,
+                                                rowof, mode, s);
   if (node_format == NODES_Q16)
     return full ? launch_nlist_f<NODES_Q16, true>(tv, radius, nl, list, offsets, out, buffer,
                                                   rowof, mode, s)

@@ -1,0 +1,102 @@
+"""Radius searches of point trees by 64 lanes together, against the oracle's
+rope walk (rows equal in order): the sizes at the edges of leaf blocks, of the
+levels above them and of wavefronts, radii and positions at which the
+half-precision test of a pair is tightest or cannot be used, and wavefronts
+whose predicates lie far apart and walk alone."""
+import numpy as np
+import pytest
+import torch
+
+import arborx_amd as ax
+import oracle
+from arborx_amd import synthetic
+
+pytestmark = pytest.mark.gpu
+
+
+def _check(points, spheres, fmt="q16", sort=True):
+    t = oracle.Tree(points, 0)
+    o_ref, i_ref = t.query_spatial(0, spheres)
+    tree = ax.BVH(torch.from_numpy(points).cuda(), node_format=fmt)
+    i, o = tree.query(ax.intersects(ax.Spheres(torch.from_numpy(spheres))),
+                      ax.TraversalPolicy(0, sort))
+    np.testing.assert_array_equal(o.cpu().numpy(), o_ref)
+    np.testing.assert_array_equal(i.cpu().numpy(), i_ref)
+    return o_ref[-1]
+
+
+def _spheres(p, r):
+    return np.concatenate([p, np.broadcast_to(np.float32(r), (len(p),)).reshape(-1, 1)],
+                          1).astype(np.float32)
+
+
+@pytest.mark.parametrize("fmt", ["fp32", "q16"])
+@pytest.mark.parametrize("n", [2, 5, 63, 64, 65, 255, 4095, 4096, 4097, 20001, 262145])
+def test_edges_of_blocks_and_levels(n, fmt):
+    p = synthetic.uniform_points(n, n % 97)
+    r = min(synthetic.radius_for_neighbours(n, 24), 0.6)
+    nq = min(n, 20001)
+    assert _check(p, _spheres(p[:nq], r), fmt) >= nq
+
+
+@pytest.mark.parametrize("nq", [1, 63, 64, 65, 1000, 4001])
+def test_edges_of_wavefronts_and_order(nq):
+    p = synthetic.uniform_points(3000, 5)
+    q = synthetic.uniform_points(nq, 6) * np.float32(1.2) - np.float32(0.1)
+    g = np.random.default_rng(nq)
+    s = _spheres(q, 0.0)
+    s[:, 3] = g.uniform(0.0, 0.12, nq)
+    for sort in (True, False):
+        _check(p, s, sort=sort)
+
+
+@pytest.mark.parametrize("scale,shift", [(1.0, 0.0), (1e-6, 0.0), (1e6, 0.0), (1.0, 1000.0),
+                                         (1e-13, 0.0), (1e16, 0.0)])
+def test_scales_and_offsets(scale, shift):
+    # a grid whose spacing is the radius: hits and misses at the threshold
+    a = np.arange(12, dtype=np.float64)
+    p = np.stack(np.meshgrid(a, a, a, indexing="ij"), -1).reshape(-1, 3) / 12.0
+    p = (p * scale + shift).astype(np.float32)
+    for k in (1.0, np.sqrt(2.0), 2.0):
+        r = np.float32(k * scale / 12.0)
+        for rr in (np.nextafter(r, np.float32(0)), r, np.nextafter(r, np.float32(np.inf))):
+            _check(p, _spheres(p, rr))
+
+
+def test_radii_and_centres_without_hits_or_bounds():
+    p = synthetic.uniform_points(5000, 1)
+    s = _spheres(p, 0.08)
+    s[::7, 3] = 0.0
+    s[3::7, 3] = -1.0
+    s[5::11, 3] = np.nan
+    s[64:128, 3] = 1e-20
+    s[777, 3] = np.inf
+    s[1000, 0] = np.nan
+    s[2000, 1] = np.inf
+    s[3000, 2] = 1e30
+    _check(p, s)
+    p[::2] = p[0]  # many duplicates: rows longer than a scratch row
+    _check(p, _spheres(p[:600], 0.01), "fp32")
+
+
+def test_far_apart_predicates_walk_alone():
+    # clusters at the corners of a large cube; wavefronts span several
+    g = np.random.default_rng(3)
+    c = np.array([[x, y, z] for x in (0, 1) for y in (0, 1) for z in (0, 1)], np.float64) * 1e4
+    p = (c[np.arange(40000) % 8] + g.normal(size=(40000, 3))).astype(np.float32)
+    _check(p, _spheres(p[g.permutation(40000)[:8000]], 0.15), sort=False)
+    _check(p, _spheres(p[:6000], 30.0)[::40].copy(), sort=False)
+
+
+@pytest.mark.parametrize("n", [2, 65, 4097, 30000])
+def test_neighbour_list_leaves_the_point_out(n):
+    p = synthetic.uniform_points(n, 8)
+    p[n // 2:n // 2 + 3] = p[0]  # duplicates of a point are its neighbours
+    r = min(synthetic.radius_for_neighbours(n, 40), 0.5)
+    # rows of the radius query without the point itself, in the same order
+    o_all, i_all = oracle.Tree(p, 0).query_spatial(0, _spheres(p, r))
+    own = np.repeat(np.arange(n), np.diff(o_all))
+    o_ref, _ = oracle.neighbor_list(p, r, True)
+    o, i = ax.find_full_neighbor_list(torch.from_numpy(p).cuda(), r)
+    np.testing.assert_array_equal(o.cpu().numpy(), o_ref)
+    np.testing.assert_array_equal(i.cpu().numpy(), i_all[i_all != own])
