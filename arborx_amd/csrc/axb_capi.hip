@@ -1525,7 +1525,10 @@ axb_status axb_bvh_query_nearest(const axb_bvh *t, const float *points, int64_t 
     {
       Region perm_region("ArborX::BVH::query::nearest::compute_permutation");
       axb_status st = predicate_order(t, err.p, PRED_RADIUS, points, nq, s, &order, &order_blk,
-                                      CURVE_MORTON24);
+                                      t->geometry == GEOM_POINTS &&
+                                              !knn_group_rule(view_of(t, err.p), nq, k)
+                                          ? CURVE_MORTON24
+                                          : CURVE_HILBERT24);
       if (st != AXB_OK)
       {
         out_free(*indices, s);

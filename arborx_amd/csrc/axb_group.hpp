@@ -279,6 +279,14 @@ AXB_D void group_exact(const GroupLds &L, uint32_t words, float x, float y, floa
                        int32_t skip, Sink &sink)
 {
   const int lane = threadIdx.x & 63;
+  if constexpr (Sink::COUNTS_ON)
+    if (sink.full())
+    {
+      // too many already: a lane that only counts takes its candidates as
+      // they are
+      for (; words; words &= words - 1u)
+        sink.cnt += __popc(L.mask[__builtin_ctz(words)][lane]);
+    }
   uint32_t mask = 0;
   const uint4 *word = L.leaf;
   while (mask | words)
@@ -292,9 +300,58 @@ AXB_D void group_exact(const GroupLds &L, uint32_t words, float x, float y, floa
     }
     const uint4 s = word[__builtin_ctz(mask)];
     mask &= mask - 1u;
-    if (dist2_pp(x, y, z, bits_f(s.x), bits_f(s.y), bits_f(s.z)) <= thr)
+    const float d2 = dist2_pp(x, y, z, bits_f(s.x), bits_f(s.y), bits_f(s.z));
+    if (d2 <= thr)
       if (!SKIP || (int32_t)s.w != ~skip)
-        sink.hit(~(int32_t)s.w);
+        sink.hit(~(int32_t)s.w, d2);
+  }
+}
+
+// Calls fn(block, leaf) for every leaf of the blocks that group_blocks found
+// (nodes of them, in L.blocks / L.node[buffer]), a block at a time and in
+// leaf order, lane l with the block's leaf l (a copy of the last leaf past
+// the end); the next block's leaves are in flight meanwhile.
+template <class Fn>
+AXB_D void group_leaves(const TreeView &tv, const GroupLds &L, int nodes, int buffer, Fn &&fn)
+{
+  const uint32_t n = (uint32_t)tv.n, lane = threadIdx.x & 63u;
+  // node `at`, its remaining blocks in `rest`
+  int at = -1;
+  uint32_t base = 0;
+  uint64_t rest = 0;
+  auto next_block = [&](uint32_t &b) {
+    while (rest == 0)
+    {
+      if (++at >= nodes)
+        return false;
+      const uint64_t m = L.blocks[at];
+      rest = (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)m) |
+             ((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(m >> 32)) << 32);
+      base = (uint32_t)__builtin_amdgcn_readfirstlane((int)L.node[buffer][at]) * 64u;
+    }
+    b = base + (uint32_t)__builtin_ctzll(rest);
+    rest &= rest - 1ull;
+    return true;
+  };
+  auto load = [&](uint32_t b) {
+    const uint32_t i = b * 64u + lane;
+    return tv.leaves[i < n ? i : n - 1];
+  };
+  uint32_t blk = 0, blk_next = 0;
+  uint4 s = make_uint4(0u, 0u, 0u, 0u);
+  bool more = next_block(blk);
+  if (more)
+    s = load(blk);
+  while (more)
+  {
+    const bool more_next = next_block(blk_next);
+    uint4 s_next = s;
+    if (more_next)
+      s_next = load(blk_next);
+    fn(blk, s);
+    s = s_next;
+    blk = blk_next;
+    more = more_next;
   }
 }
 
@@ -322,42 +379,9 @@ AXB_D bool group_walk(const TreeView &tv, GroupLds &L, float x, float y, float z
   group_columns(g, x, y, z, r, active, col);
   const int lane = threadIdx.x & 63;
   const uint32_t n = (uint32_t)tv.n;
-  // the leaf blocks in order: node `at`, its remaining blocks in `rest`
-  int at = -1;
-  uint32_t base = 0;
-  uint64_t rest = 0;
-  auto next_block = [&](uint32_t &b) {
-    while (rest == 0)
-    {
-      if (++at >= nodes)
-        return false;
-      const uint64_t m = L.blocks[at];
-      rest = (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)m) |
-             ((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(m >> 32)) << 32);
-      base = (uint32_t)__builtin_amdgcn_readfirstlane((int)L.node[buffer][at]) * 64u;
-    }
-    b = base + (uint32_t)__builtin_ctzll(rest);
-    rest &= rest - 1ull;
-    return true;
-  };
-  auto load = [&](uint32_t b) {
-    const uint32_t i = b * 64u + (uint32_t)lane;
-    return tv.leaves[i < n ? i : n - 1];
-  };
   int cnt = 0, done = 0; // candidates in LDS, and those whose masks are made
   uint32_t words = 0;
-  uint32_t blk = 0, blk_next = 0;
-  uint4 s = make_uint4(0u, 0u, 0u, 0u);
-  bool more = next_block(blk);
-  if (more)
-    s = load(blk);
-  while (more)
-  {
-    // the next block's leaves are in flight while this block is tested
-    const bool more_next = next_block(blk_next);
-    uint4 s_next = s;
-    if (more_next)
-      s_next = load(blk_next);
+  group_leaves(tv, L, nodes, buffer, [&](uint32_t blk, uint4 s) {
     ++v_leaf;
     const bool in = blk * 64u + (uint32_t)lane < n &&
                     group_point_d2(g, bits_f(s.x), bits_f(s.y), bits_f(s.z)) <= g.thr;
@@ -391,10 +415,7 @@ AXB_D bool group_walk(const TreeView &tv, GroupLds &L, float x, float y, float z
         wave_lds_order();
       }
     }
-    s = s_next;
-    blk = blk_next;
-    more = more_next;
-  }
+  });
   if (cnt > done)
   {
     // the last, partial word: its bits past the candidates are dropped
@@ -404,6 +425,67 @@ AXB_D bool group_walk(const TreeView &tv, GroupLds &L, float x, float y, float z
   }
   group_exact<SKIP>(L, words, x, y, z, thr, skip, sink);
   return true;
+}
+
+// ------------------------------------------------------------ nearest
+// The radius within which a lane should find about `want` leaves, from the
+// leaves in and just around the group's box: their number over the volume
+// they were counted in gives the density, and a ball that reaches beyond the
+// scene box is enlarged for the part outside.  A guess: the caller counts
+// what it finds.  spacing: about the distance between leaves.  False when
+// the group's box holds too many blocks.
+AXB_D bool group_guess_radius(const TreeView &tv, GroupLds &L, float x, float y, float z,
+                              bool active, float want, float spacing, float &r, uint32_t &v_int,
+                              uint32_t &v_leaf)
+{
+  GroupReach g;
+  if (!group_reach(x, y, z, 0.f, 0.f, active, g))
+  {
+    // all centres in one place (or none that can be searched)
+    const float h = wave_uniform(wave_max(active ? fabsf(x) + fabsf(y) + fabsf(z) : 0.f));
+    if (!(h < 1e15f))
+      return false;
+  }
+  const float ex = g.hi[0] - g.lo[0], ey = g.hi[1] - g.lo[1], ez = g.hi[2] - g.lo[2];
+  float grow = 0.1f * fmaxf(fmaxf(ex, ey), ez);
+  const uint32_t n = (uint32_t)tv.n, lane = threadIdx.x & 63u;
+  int found = 0;
+  for (int t = 0;; ++t)
+  {
+    g.thr = grow * grow;
+    int buffer = 0;
+    const int nodes = group_blocks(tv, g, L, buffer, v_int);
+    if (nodes < 0)
+      return false;
+    found = 0;
+    group_leaves(tv, L, nodes, buffer, [&](uint32_t blk, uint4 s) {
+      ++v_leaf;
+      found += __popcll(__ballot(
+          blk * 64u + lane < n &&
+          group_point_d2(g, bits_f(s.x), bits_f(s.y), bits_f(s.z)) <= g.thr));
+    });
+    wave_lds_order();
+    if (found >= 24 || t == 5)
+      break;
+    grow = fmaxf(2.f * grow, 0.5f * spacing);
+  }
+  const float vol = ex * ey * ez + 2.f * grow * (ex * ey + ey * ez + ez * ex) +
+                    3.14159265f * grow * grow * (ex + ey + ez) + 4.18879f * grow * grow * grow;
+  // cube roots by exp2(log2 / 3): only a guess
+  const float third = 1.f / 3.f;
+  const float r0 = __builtin_amdgcn_exp2f(
+      third * __builtin_amdgcn_logf(0.238732f * want * vol / (float)(found > 0 ? found : 1)));
+  float in = 1.f;
+  const float c[3] = {x, y, z};
+#pragma unroll
+  for (int d = 0; d < 3; ++d)
+  {
+    const float gap = fmaxf(fminf(c[d] - tv.scene.lo[d], tv.scene.hi[d] - c[d]), 0.f);
+    const float u = fminf(gap / r0, 1.f); // part of the ball's axis inside
+    in *= 0.5f + 0.5f * u * (1.5f - 0.5f * u * u);
+  }
+  r = r0 * __builtin_amdgcn_exp2f(-third * __builtin_amdgcn_logf(in));
+  return wave_uniform(r0) > 0.f && r0 < 1e15f;
 }
 
 } // namespace axb

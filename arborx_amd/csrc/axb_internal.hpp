@@ -279,6 +279,9 @@ struct RowWriter
     ++cnt;
     return true;
   }
+  // (the group walk's hits carry their squared distance)
+  static constexpr bool COUNTS_ON = false;
+  AXB_D bool hit(int32_t v, float) { return hit(v); }
   // Writes the last partial group of the hits (nothing for a row that
   // overflowed: its count sends it to be walked again).
   AXB_D void finish()
@@ -422,14 +425,19 @@ hipError_t launch_knn(const TreeView &tv, int node_format, int geometry, const f
                       hipStream_t s);
 // Buffers of a kNN call for k <= 64: candidate rows for `batch` queries
 // (batch * knn_row_capacity(k, n) entries, batch * capacity + capacity
-// below 2^32), the list of unresolved queries (nq entries) and its counter.
+// below 2^32), the list of unresolved queries (nq entries), its counter and
+// the counter of the list of what the group search left (null: no such
+// search).
 struct KnnScratch
 {
   uint2 *cand;
   int64_t batch;
   uint32_t *ovf;
-  uint32_t *ovf_n;
+  uint32_t *ovf_n; // two words
+  uint32_t *left;
 };
+// Whether queries in Hilbert order are searched in groups.
+bool knn_group_rule(const TreeView &tv, int64_t nq, int k);
 int knn_row_capacity(int k, int n);
 hipError_t launch_knn_offsets(int64_t *offsets, int64_t nq, int64_t per, hipStream_t s);
 // keys = the predicates' 30-bit Morton codes, their top 24 bits, or 24-bit

@@ -1062,14 +1062,15 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu((K <= 16 &&
     TreeView tv, const float *__restrict__ pts, int64_t t0, int64_t tn, int k, int W,
     const uint32_t *__restrict__ order, uint2 *__restrict__ cand, int cap, float shrink,
     int max_rounds, uint32_t *__restrict__ ovf, uint32_t *__restrict__ ovf_n,
-    int32_t *__restrict__ oi, float *__restrict__ od)
+    int32_t *__restrict__ oi, float *__restrict__ od, const uint32_t *__restrict__ list,
+    const uint32_t *__restrict__ list_n)
 {
   __shared__ __align__(16) uint2 s_stage[G == GEOM_POINTS ? KNN_STAGE * 256 : 1];
   const int64_t g = (int64_t)xcd_block(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
-  if (g >= tn)
+  if (g >= tn || (list && t0 + g >= (int64_t)*list_n))
     return;
   CandStage stage{s_stage, (int)threadIdx.x};
-  const int64_t t = t0 + g;
+  const int64_t t = list ? (int64_t)list[t0 + g] : t0 + g;
   const int64_t q = order ? (int64_t)order[t] : t;
   const float qx = pts[3 * q], qy = pts[3 * q + 1], qz = pts[3 * q + 2];
   const int m = k < tv.n ? k : tv.n;
@@ -1114,6 +1115,146 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu((K <= 16 &&
   if (COUNT && tv.visits)
   {
     atomicAdd(tv.visits + 0, 1ull);
+    atomicAdd(tv.visits + 1, (unsigned long long)v_int);
+    atomicAdd(tv.visits + 2, (unsigned long long)v_leaf);
+    atomicAdd(tv.visits + 3, (unsigned long long)c);
+    atomicAdd(tv.visits + 8, (unsigned long long)rounds);
+    if (rounds > 1)
+      atomicAdd(tv.visits + 9, 1ull);
+  }
+}
+
+// Candidate row of a group's lane: {index, d2 bits} pairs written two per
+// 16-byte store; beyond `cap` entries it only counts.
+struct GroupCand
+{
+  static constexpr bool COUNTS_ON = true;
+  uint2 *__restrict__ cand;
+  uint32_t row_at;
+  int cap, cnt;
+  uint2 held;
+  AXB_D bool full() const { return cnt > cap; }
+  AXB_D void hit(int32_t v, float d2)
+  {
+    const uint2 e = make_uint2((uint32_t)v, f_bits(d2));
+    if ((cnt & 1) && cnt < cap)
+      *reinterpret_cast<uint4 *>(cand + row_at + (uint32_t)(cnt - 1)) =
+          make_uint4(held.x, held.y, e.x, e.y);
+    held = e;
+    ++cnt;
+  }
+  AXB_D void finish()
+  {
+    if ((cnt & 1) && cnt <= cap)
+      cand[row_at + (uint32_t)(cnt - 1)] = held;
+  }
+};
+
+// Distance of the m-th nearest of the first `cap` entries of a full row (cap
+// a multiple of 8): they are real leaves, so the m-th nearest leaf is no
+// farther, and a search within it finds at least m.
+template <int K>
+AXB_D float group_row_bound(const uint2 *__restrict__ cand, uint32_t row_at, int cap, int m)
+{
+  constexpr int NB = K < 8 ? K : 8;
+  uint32_t A[K];
+#pragma unroll
+  for (int j = 0; j < K; ++j)
+    A[j] = j < K - m ? 0u : ~0u; // the m-th smallest is A[K - 1]
+#pragma unroll 1
+  for (int b = 0; b < cap; b += NB)
+  {
+    uint32_t B[NB];
+#pragma unroll
+    for (int j = 0; j < NB; ++j)
+      B[j] = cand[row_at + (uint32_t)(b + j)].y;
+    bitonic_sort<NB>(B);
+#pragma unroll
+    for (int j = K - NB; j < K; ++j)
+      A[j] = A[j] < B[K - 1 - j] ? A[j] : B[K - 1 - j];
+    bitonic_merge<K>(A);
+  }
+  return sqrt_rn(bits_f(A[K - 1]));
+}
+
+// k nearest of points that are neighbours along the Hilbert curve, 64 lanes
+// searching together (axb_group.hpp): a radius is guessed from the density
+// of the leaves around the group (no descent, no seed window), the group
+// walk gathers every leaf within it in the lanes' candidate rows, and a
+// lane whose row holds between m and cap of them selects its m nearest; the
+// others search again together: a short row with a larger radius, from its
+// count, a full one within its m-th distance.
+// What is left after GROUP_ROUNDS goes to the list for k_knn_collect.
+constexpr int GROUP_ROUNDS = 6;
+template <int K, bool COUNT>
+__global__ __launch_bounds__(256, K <= 16 ? 5 : (K <= 32 ? 4 : 2)) void k_knn_group(
+    TreeView tv, const float *__restrict__ pts, int64_t t0, int64_t tn, int k, float want,
+    float spacing, const uint32_t *__restrict__ order, uint2 *__restrict__ cand, int cap,
+    int max_rounds, uint32_t *__restrict__ left, uint32_t *__restrict__ left_n,
+    int32_t *__restrict__ oi, float *__restrict__ od)
+{
+  __shared__ GroupLds s_group[4];
+  const int64_t g = (int64_t)xcd_block(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
+  const bool real = g < tn;
+  const int64_t t = t0 + g;
+  int64_t q = 0;
+  float x = 0.f, y = 0.f, z = 0.f;
+  if (real)
+  {
+    q = (int64_t)order[t];
+    x = pts[3 * q], y = pts[3 * q + 1], z = pts[3 * q + 2];
+  }
+  const int m = k < tv.n ? k : tv.n;
+  GroupLds &L = s_group[threadIdx.x >> 6];
+  bool pending = real && fabsf(x) < INFINITY && fabsf(y) < INFINITY && fabsf(z) < INFINITY;
+  uint32_t v_int = 0, v_leaf = 0;
+  GroupCand row{cand, real ? (uint32_t)(g * cap) : 0u, cap, 0, make_uint2(0u, 0u)};
+  int c = 0, rounds = 0;
+  float r = 0.f;
+  if (max_rounds > 0 &&
+      group_guess_radius(tv, L, x, y, z, pending, want, spacing, r, v_int, v_leaf))
+  {
+#pragma unroll 1
+    for (int round = 0; round < (max_rounds < GROUP_ROUNDS ? max_rounds : GROUP_ROUNDS); ++round)
+    {
+      if (__ballot(pending) == 0)
+        break;
+      ++rounds;
+      row.cnt = 0;
+      if (!group_walk<false>(tv, L, x, y, z, r, sqrt_threshold(r), pending, -1, row, v_int,
+                             v_leaf))
+        break;
+      if (pending)
+      {
+        if (row.cnt >= m && row.cnt <= cap)
+        {
+          row.finish();
+          c = row.cnt;
+          pending = false;
+        }
+        else if (row.cnt < m)
+        {
+          const float f = __builtin_amdgcn_exp2f(
+              (1.f / 3.f) *
+              __builtin_amdgcn_logf(want / (float)(row.cnt > 0 ? row.cnt : 1)));
+          r *= fminf(fmaxf(f, 1.26f), 2.5f);
+        }
+      }
+      if (__ballot(pending && row.cnt > cap))
+      {
+        const float bound = group_row_bound<K>(cand, row.row_at, cap, m);
+        if (pending && row.cnt > cap)
+          r = bound;
+      }
+    }
+  }
+  if (c > 0) // exact top-m of the row (every leaf within the m-th distance is in it)
+    select_row<K>(cand, row.row_at, c, m, oi, od, q * m);
+  else if (real)
+    left[atomicAdd(left_n, 1u)] = (uint32_t)t;
+  if (COUNT && tv.visits && real)
+  {
+    atomicAdd(tv.visits + 0, c > 0 ? 1ull : 0ull); // the others are counted by k_knn_collect
     atomicAdd(tv.visits + 1, (unsigned long long)v_int);
     atomicAdd(tv.visits + 2, (unsigned long long)v_leaf);
     atomicAdd(tv.visits + 3, (unsigned long long)c);
@@ -1570,6 +1711,17 @@ static KnnShape knn_shape(int k, int n)
 
 int knn_row_capacity(int k, int n) { return knn_shape(k, n).cap; }
 
+// Leaves the group search aims at for k nearest: a count that is Poisson
+// around k + 4 sqrt(k) + 4 falls below k once in ~10^4.
+static float knn_group_want(int k) { return (float)k + 4.f * std::sqrt((float)k) + 4.f; }
+// Queries of a point tree that are sorted along the Hilbert curve search in
+// groups when they are not far fewer than the points.
+bool knn_group_rule(const TreeView &tv, int64_t nq, int k)
+{
+  return tv.leaves && k >= 1 && k <= 64 && nq * 8 >= tv.n &&
+         (float)tv.n >= 8.f * knn_group_want(k);
+}
+
 template <int F, int G, int K>
 static hipError_t knn_run(const TreeView &tv, const float *pts, int64_t nq, int k,
                           const uint32_t *order, int32_t *oi, float *od, const KnnScratch &ws,
@@ -1578,17 +1730,46 @@ static hipError_t knn_run(const TreeView &tv, const float *pts, int64_t nq, int 
   const KnnShape sh = knn_shape(k, tv.n);
   const int lim = debug_limits().knn_rounds;
   const int rounds = lim > 0 ? lim : (lim < 0 ? 0 : KNN_ROUNDS);
-  hipError_t e = fill_u32(ws.ovf_n, 0u, 1, s);
+  hipError_t e = fill_u32(ws.ovf_n, 0u, 2, s);
+  // points: the group walk first; the list of what it left goes through
+  // the collect launches below
+  const uint32_t *list = nullptr, *list_n = nullptr;
+  if constexpr (G == GEOM_POINTS)
+    if (ws.left)
+    {
+      const float want = knn_group_want(k);
+      float vol = 1.f, longest = 0.f;
+      for (int d = 0; d < 3; ++d)
+        longest = std::max(longest, tv.scene.hi[d] - tv.scene.lo[d]);
+      for (int d = 0; d < 3; ++d)
+        vol *= std::max(tv.scene.hi[d] - tv.scene.lo[d], 1e-3f * longest);
+      const float spacing = std::cbrt(vol / (float)tv.n);
+      for (int64_t t0 = 0; e == hipSuccess && t0 < nq; t0 += ws.batch)
+      {
+        const int64_t tn = std::min(ws.batch, nq - t0);
+        if (tv.visits)
+          AXB_LAUNCH((k_knn_group<K, true>), dim3(grid_of(tn)), dim3(256), 0, s, tv, pts, t0, tn,
+                     k, want, spacing, order, ws.cand, sh.cap, rounds, ws.left, ws.ovf_n + 1, oi,
+                     od);
+        else
+          AXB_LAUNCH((k_knn_group<K, false>), dim3(grid_of(tn)), dim3(256), 0, s, tv, pts, t0,
+                     tn, k, want, spacing, order, ws.cand, sh.cap, rounds, ws.left, ws.ovf_n + 1,
+                     oi, od);
+        e = hipGetLastError();
+      }
+      list = ws.left, list_n = ws.ovf_n + 1;
+    }
   for (int64_t t0 = 0; e == hipSuccess && t0 < nq; t0 += ws.batch)
   {
     const int64_t tn = std::min(ws.batch, nq - t0);
     if (tv.visits)
       AXB_LAUNCH((k_knn_collect<F, G, K, true>), dim3(grid_of(tn)), dim3(256), 0, s, tv, pts, t0,
-                 tn, k, sh.W, order, ws.cand, sh.cap, sh.shrink, rounds, ws.ovf, ws.ovf_n, oi, od);
+                 tn, k, sh.W, order, ws.cand, sh.cap, sh.shrink, rounds, ws.ovf, ws.ovf_n, oi, od,
+                 list, list_n);
     else
       AXB_LAUNCH((k_knn_collect<F, G, K, false>), dim3(grid_of(tn)), dim3(256), 0, s, tv, pts,
                  t0, tn, k, sh.W, order, ws.cand, sh.cap, sh.shrink, rounds, ws.ovf, ws.ovf_n, oi,
-                 od);
+                 od, list, list_n);
     e = hipGetLastError();
   }
   // unresolved queries of every batch, in one launch at the end: each of
@@ -1628,12 +1809,17 @@ static hipError_t knn_pipeline(const TreeView &tv, const float *pts, int64_t nq,
     batch = (batch + 1) / 2;
   }
   KnnScratch ws{(uint2 *)rows.p, batch, (uint32_t *)dalloc((size_t)nq * sizeof(uint32_t), s),
-                (uint32_t *)dalloc(sizeof(uint32_t), s)};
-  hipError_t e = (ws.cand && ws.ovf && ws.ovf_n) ? hipSuccess : hipErrorOutOfMemory;
+                (uint32_t *)dalloc(2 * sizeof(uint32_t), s), nullptr};
+  const bool group = G == GEOM_POINTS && order && knn_group_rule(tv, nq, k);
+  if (group)
+    ws.left = (uint32_t *)dalloc((size_t)nq * sizeof(uint32_t), s);
+  hipError_t e = (ws.cand && ws.ovf && ws.ovf_n && (!group || ws.left)) ? hipSuccess
+                                                                        : hipErrorOutOfMemory;
   if (e == hipSuccess)
     e = knn_run<F, G, K>(tv, pts, nq, k, order, oi, od, ws, s);
   dfree(ws.ovf, s);
   dfree(ws.ovf_n, s);
+  dfree(ws.left, s);
   return e;
 }
 

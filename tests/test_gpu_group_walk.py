@@ -100,3 +100,63 @@ def test_neighbour_list_leaves_the_point_out(n):
     o, i = ax.find_full_neighbor_list(torch.from_numpy(p).cuda(), r)
     np.testing.assert_array_equal(o.cpu().numpy(), o_ref)
     np.testing.assert_array_equal(i.cpu().numpy(), i_all[i_all != own])
+
+
+# ------------------------------------------------------------ nearest
+def _check_nearest(points, queries, k, fmt="q16"):
+    t = oracle.Tree(points, 0)
+    o_ref, i_ref, d_ref = t.query_knn(queries, k)
+    tree = ax.BVH(torch.from_numpy(points).cuda(), node_format=fmt)
+    i, o, d = tree.query(ax.make_nearest(torch.from_numpy(queries), k), return_distances=True)
+    np.testing.assert_array_equal(o.cpu().numpy(), o_ref)
+    np.testing.assert_array_equal(i.cpu().numpy(), i_ref)
+    np.testing.assert_array_equal(d.cpu().numpy().view(np.uint32), d_ref.view(np.uint32))
+
+
+@pytest.mark.parametrize("fmt", ["fp32", "q16"])
+@pytest.mark.parametrize("k", [1, 2, 3, 5, 8, 13, 16, 17, 32, 33, 64])
+def test_nearest_uniform(k, fmt):
+    p = synthetic.uniform_points(5000, k)
+    _check_nearest(p, p, k, fmt)
+    q = synthetic.uniform_points(1001, k + 100) * np.float32(1.5) - np.float32(0.25)
+    _check_nearest(p, q, k, fmt)
+
+
+@pytest.mark.parametrize("k", [1, 10, 40])
+def test_nearest_uneven_density(k):
+    g = np.random.default_rng(k)
+    n = 12000
+    # clusters of very different widths, a line, a plane, duplicates, outliers
+    p = g.uniform(size=(n, 3))
+    w = 10.0 ** g.uniform(-4, -1, 40)
+    c = g.uniform(size=(40, 3))
+    i = np.arange(6000) % 40
+    p[:6000] = c[i] + w[i, None] * g.normal(size=(6000, 3))
+    p[6000:7500, 1:] = 0.5
+    p[7500:9000, 2] = 0.25
+    p[9000:9200] = p[9000]
+    p[9200:9210] *= 50.0
+    p = p.astype(np.float32)
+    _check_nearest(p, p, k)
+    _check_nearest(p, np.roll(p, 1, axis=1)[:3000].copy(), k)
+    _check_nearest(p, np.repeat(p[8990:9010], 200, axis=0), k)
+
+
+def test_nearest_ties_and_lists_of_queries_left():
+    a = np.arange(18, dtype=np.float32)
+    p = np.stack(np.meshgrid(a, a, a, indexing="ij"), -1).reshape(-1, 3)
+    _check_nearest(p, p, 16)  # a grid: the 16th is tied with others
+    q = synthetic.uniform_points(4000, 2)
+    q[::9, 0] = np.nan
+    q[1::9] = 3e18
+    ref = ax.BruteForce(torch.from_numpy(p).cuda()).query(
+        ax.make_nearest(torch.from_numpy(q), 6), return_distances=True)
+    tree = ax.BVH(torch.from_numpy(p).cuda())
+    for kw in (dict(), dict(knn_batch_max=777), dict(knn_rounds=1), dict(knn_rounds=-1)):
+        with ax.debug_limits(**kw):
+            got = tree.query(ax.make_nearest(torch.from_numpy(q), 6), return_distances=True)
+        keep = torch.from_numpy(~np.isnan(q[:, 0])).cuda()
+        for x, y in zip(got, ref):
+            if x.numel() == 6 * len(q):
+                x, y = x.reshape(-1, 6)[keep], y.reshape(-1, 6)[keep]
+            assert torch.equal(x, y), kw
