@@ -163,9 +163,11 @@ AXB_D bool group_reach(float x, float y, float z, float r, float thr, bool activ
 // Leaf blocks within reach: L.blocks[j] has bit b set for block 64 node[j] +
 // b, nodes in leaf order (node = L.node[the returned buffer]).  Returns the
 // number of nodes, or -1 when more blocks or nodes are within reach than a
-// group may look at.
+// group may look at.  see(m, a, b): the mask of the blocks within reach below
+// a node, lane l with the box of block l.
+template <class See>
 AXB_D int group_blocks(const TreeView &tv, const GroupReach &g, GroupLds &L, int &buffer,
-                       uint32_t &tested)
+                       uint32_t &tested, See &&see)
 {
   const int lane = threadIdx.x & 63;
   int cnt = 1, cur = 0;
@@ -182,8 +184,12 @@ AXB_D int group_blocks(const TreeView &tv, const GroupReach &g, GroupLds &L, int
       const uint32_t id = (uint32_t)__builtin_amdgcn_readfirstlane((int)L.node[cur][j]) * 64u +
                           (uint32_t)lane;
       bool in = false;
+      float4 a = make_float4(0.f, 0.f, 0.f, 0.f), b = a;
       if (id < total)
-        in = group_box_d2(g, boxes[2 * (size_t)id], boxes[2 * (size_t)id + 1]) <= g.thr;
+      {
+        a = boxes[2 * (size_t)id], b = boxes[2 * (size_t)id + 1];
+        in = group_box_d2(g, a, b) <= g.thr;
+      }
       ++tested;
       const uint64_t m = __ballot(in);
       const int more = __popcll(m);
@@ -193,6 +199,7 @@ AXB_D int group_blocks(const TreeView &tv, const GroupReach &g, GroupLds &L, int
       {
         if (lane == 0)
           L.blocks[j] = m;
+        see(m, a, b);
       }
       else if (in)
         L.node[cur ^ 1][got + (int)lanes_below(m)] = id;
@@ -372,7 +379,8 @@ AXB_D bool group_walk(const TreeView &tv, GroupLds &L, float x, float y, float z
   if (!group_reach(x, y, z, r, thr, active, g))
     return false;
   int buffer = 0;
-  const int nodes = group_blocks(tv, g, L, buffer, v_int);
+  const int nodes =
+      group_blocks(tv, g, L, buffer, v_int, [](uint64_t, const float4 &, const float4 &) {});
   if (nodes < 0)
     return false;
   half4_t col[2];
@@ -428,24 +436,24 @@ AXB_D bool group_walk(const TreeView &tv, GroupLds &L, float x, float y, float z
 }
 
 // ------------------------------------------------------------ nearest
+AXB_D float approx_cbrt(float v) // exp2(log2 / 3): for guesses only
+{
+  return __builtin_amdgcn_exp2f((1.f / 3.f) * __builtin_amdgcn_logf(v));
+}
+
 // The radius within which a lane should find about `want` leaves, from the
 // leaves in and just around the group's box: their number over the volume
 // they were counted in gives the density, and a ball that reaches beyond the
 // scene box is enlarged for the part outside.  A guess: the caller counts
 // what it finds.  spacing: about the distance between leaves.  False when
-// the group's box holds too many blocks.
+// the box holds too many blocks or there is nothing to go by.
 AXB_D bool group_guess_radius(const TreeView &tv, GroupLds &L, float x, float y, float z,
                               bool active, float want, float spacing, float &r, uint32_t &v_int,
                               uint32_t &v_leaf)
 {
   GroupReach g;
   if (!group_reach(x, y, z, 0.f, 0.f, active, g))
-  {
-    // all centres in one place (or none that can be searched)
-    const float h = wave_uniform(wave_max(active ? fabsf(x) + fabsf(y) + fabsf(z) : 0.f));
-    if (!(h < 1e15f))
-      return false;
-  }
+    return false; // all centres in one place
   const float ex = g.hi[0] - g.lo[0], ey = g.hi[1] - g.lo[1], ez = g.hi[2] - g.lo[2];
   float grow = 0.1f * fmaxf(fmaxf(ex, ey), ez);
   const uint32_t n = (uint32_t)tv.n, lane = threadIdx.x & 63u;
@@ -454,7 +462,8 @@ AXB_D bool group_guess_radius(const TreeView &tv, GroupLds &L, float x, float y,
   {
     g.thr = grow * grow;
     int buffer = 0;
-    const int nodes = group_blocks(tv, g, L, buffer, v_int);
+    const int nodes =
+      group_blocks(tv, g, L, buffer, v_int, [](uint64_t, const float4 &, const float4 &) {});
     if (nodes < 0)
       return false;
     found = 0;
@@ -471,10 +480,7 @@ AXB_D bool group_guess_radius(const TreeView &tv, GroupLds &L, float x, float y,
   }
   const float vol = ex * ey * ez + 2.f * grow * (ex * ey + ey * ez + ez * ex) +
                     3.14159265f * grow * grow * (ex + ey + ez) + 4.18879f * grow * grow * grow;
-  // cube roots by exp2(log2 / 3): only a guess
-  const float third = 1.f / 3.f;
-  const float r0 = __builtin_amdgcn_exp2f(
-      third * __builtin_amdgcn_logf(0.238732f * want * vol / (float)(found > 0 ? found : 1)));
+  const float r0 = approx_cbrt(0.238732f * want * vol / (float)(found > 0 ? found : 1));
   float in = 1.f;
   const float c[3] = {x, y, z};
 #pragma unroll
@@ -484,8 +490,66 @@ AXB_D bool group_guess_radius(const TreeView &tv, GroupLds &L, float x, float y,
     const float u = fminf(gap / r0, 1.f); // part of the ball's axis inside
     in *= 0.5f + 0.5f * u * (1.5f - 0.5f * u * u);
   }
-  r = r0 * __builtin_amdgcn_exp2f(-third * __builtin_amdgcn_logf(in));
+  r = r0 / approx_cbrt(in);
   return wave_uniform(r0) > 0.f && r0 < 1e15f;
+}
+
+// The same from the lane's own density: every leaf block spreads its 64
+// leaves over its box, and what falls into a cube around the lane's centre
+// counts (the boxes of Morton blocks overlap, but each spreads its own leaves
+// only).  Follows a density that differs between the lanes of a group, and
+// reads no leaves, but is less exact where it does not.  per_query: leaves
+// per predicate, which sets the cube's size.
+AXB_D float lane_value(float v, int lane)
+{
+  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), lane));
+}
+AXB_D bool group_guess_own_radius(const TreeView &tv, GroupLds &L, float x, float y, float z,
+                                  bool active, float want, float per_query, float &r,
+                                  uint32_t &v_int)
+{
+  GroupReach g;
+  if (!group_reach(x, y, z, 0.f, 0.f, active, g))
+    return false;
+  const float e[3] = {g.hi[0] - g.lo[0], g.hi[1] - g.lo[1], g.hi[2] - g.lo[2]};
+  const float least = 0.2f * fmaxf(fmaxf(e[0], e[1]), e[2]);
+  const float vol = fmaxf(e[0], least) * fmaxf(e[1], least) * fmaxf(e[2], least);
+  // half the side of a cube of about want / 2 leaves, if the group's box
+  // holds per_query for each of its predicates
+  const float h = 0.5f * approx_cbrt(0.5f * want * vol /
+                                     ((float)__popcll(__ballot(active)) * per_query));
+  g.thr = h * h;
+  const float lo[3] = {x - h, y - h, z - h}, hi[3] = {x + h, y + h, z + h};
+  float mass = 0.f;
+  int buffer = 0;
+  const int nodes = group_blocks(
+      tv, g, L, buffer, v_int, [&](uint64_t m, const float4 &a, const float4 &b) {
+        // per axis: 1 / extent, 0 for a flat box
+        const float ix = a.w > a.x ? __builtin_amdgcn_rcpf(a.w - a.x) : 0.f;
+        const float iy = b.x > a.y ? __builtin_amdgcn_rcpf(b.x - a.y) : 0.f;
+        const float iz = b.y > a.z ? __builtin_amdgcn_rcpf(b.y - a.z) : 0.f;
+        for (uint64_t rest = m; rest; rest &= rest - 1ull)
+        {
+          const int l = __builtin_ctzll(rest);
+          const float bl[3] = {lane_value(a.x, l), lane_value(a.y, l), lane_value(a.z, l)};
+          const float bh[3] = {lane_value(a.w, l), lane_value(b.x, l), lane_value(b.y, l)};
+          const float bi[3] = {lane_value(ix, l), lane_value(iy, l), lane_value(iz, l)};
+          float part = 1.f;
+#pragma unroll
+          for (int d = 0; d < 3; ++d)
+          {
+            const float cut = fminf(hi[d], bh[d]) - fmaxf(lo[d], bl[d]);
+            part *= bi[d] > 0.f ? fmaxf(cut, 0.f) * bi[d] : (cut >= 0.f ? 1.f : 0.f);
+          }
+          mass += part;
+        }
+      });
+  wave_lds_order();
+  if (nodes < 0)
+    return false;
+  // 64 mass leaves in the cube of volume 8 h^3
+  r = h * approx_cbrt(want * 1.909859f / fmaxf(64.f * mass, 0.05f * want));
+  return wave_uniform(h) > 0.f && h < 1e15f;
 }
 
 } // namespace axb

@@ -425,16 +425,13 @@ hipError_t launch_knn(const TreeView &tv, int node_format, int geometry, const f
                       hipStream_t s);
 // Buffers of a kNN call for k <= 64: candidate rows for `batch` queries
 // (batch * knn_row_capacity(k, n) entries, batch * capacity + capacity
-// below 2^32), the list of unresolved queries (nq entries), its counter and
-// the counter of the list of what the group search left (null: no such
-// search).
+// below 2^32), the list of unresolved queries (nq entries) and its counter.
 struct KnnScratch
 {
   uint2 *cand;
   int64_t batch;
   uint32_t *ovf;
-  uint32_t *ovf_n; // two words
-  uint32_t *left;
+  uint32_t *ovf_n;
 };
 // Whether queries in Hilbert order are searched in groups.
 bool knn_group_rule(const TreeView &tv, int64_t nq, int k);

@@ -107,13 +107,12 @@ __global__ __launch_bounds__(256, 6) void k_spatial_group(
   if (real)
     rw.init(out, offsets, q, buffer);
   uint32_t v_int = 0, v_leaf = 0;
-  if (!group_walk<false>(tv, s_group[threadIdx.x >> 6], x, y, z, r, thr, active, -1, rw, v_int, v_leaf))
+  if (!group_walk<false>(tv, s_group[threadIdx.x >> 6], x, y, z, r, thr, active, -1, rw, v_int,
+                         v_leaf) &&
+      real)
   {
-    if (real)
-    {
-      const SpatialPred pr = sphere_pred(x, y, z, r);
-      rope_walk<F, GEOM_POINTS, PK>(tv, pr, 0u, tv.total, ~0u, rw, v_int, v_leaf);
-    }
+    const SpatialPred pr = sphere_pred(x, y, z, r);
+    rope_walk<F, GEOM_POINTS, PK>(tv, pr, 0u, tv.total, ~0u, rw, v_int, v_leaf);
   }
   if (real)
     row_epilogue(tv, rw, offsets, q, COUNT ? v_int : 0u, COUNT ? v_leaf : 0u);
@@ -342,15 +341,13 @@ __global__ __launch_bounds__(256, 6) void k_nlist_group(TreeView tv, float radiu
       real && fabsf(x) < INFINITY && fabsf(y) < INFINITY && fabsf(z) < INFINITY;
   uint32_t v_int = 0, v_leaf = 0;
   if (!group_walk<true>(tv, s_group[threadIdx.x >> 6], x, y, z, radius, thr, active, (int32_t)q,
-                        rw, v_int, v_leaf))
+                        rw, v_int, v_leaf) &&
+      real)
   {
-    if (real)
-    {
-      constexpr uint32_t SL = leaf_slots<GEOM_POINTS>(), SI = internal_slots<F>();
-      const uint32_t self = SL * L + SI * (uint32_t)tv.C[L];
-      const SpatialPred pr = sphere_pred(x, y, z, radius);
-      rope_walk<F, GEOM_POINTS, PRED_SPHERES>(tv, pr, 0u, tv.total, self, rw, v_int, v_leaf);
-    }
+    constexpr uint32_t SL = leaf_slots<GEOM_POINTS>(), SI = internal_slots<F>();
+    const uint32_t self = SL * L + SI * (uint32_t)tv.C[L];
+    const SpatialPred pr = sphere_pred(x, y, z, radius);
+    rope_walk<F, GEOM_POINTS, PRED_SPHERES>(tv, pr, 0u, tv.total, self, rw, v_int, v_leaf);
   }
   if (real)
     row_epilogue(tv, rw, offsets, q, v_int, v_leaf);
@@ -867,17 +864,18 @@ AXB_D float knn_seed(const TreeView &tv, float qx, float qy, float qz, int k, in
 // (d2, index) key, d2 bits high (d2 >= 0, so bit order is value order).  Stops as soon as more than `cap` leaves qualify;
 // returns the count (cap + 1 on overflow).
 // Candidates of a point walk gather in LDS, KNN_STAGE per lane (entry j of
-// lane l at st[j * 256 + l]), and leave for the row as whole 64-byte
+// lane l at st[j * STRIDE + l]), and leave for the row as whole 64-byte
 // chunks: each chunk of the row is written once, complete (a row's lanes
 // write far apart, so single 8-byte stores left most of each 128-byte line
 // to be written back partially, several times).
 constexpr int KNN_STAGE = 8;
+template <int STRIDE>
 struct CandStage
 {
   uint2 *st;
   int lane;
-  AXB_D void put(int c, uint2 e) { st[(c & (KNN_STAGE - 1)) * 256 + lane] = e; }
-  AXB_D uint2 get(int c) const { return st[(c & (KNN_STAGE - 1)) * 256 + lane]; }
+  AXB_D void put(int c, uint2 e) { st[(c & (KNN_STAGE - 1)) * STRIDE + lane] = e; }
+  AXB_D uint2 get(int c) const { return st[(c & (KNN_STAGE - 1)) * STRIDE + lane]; }
   // the chunk holding entries [c0, c0 + 8) of the row, c0 a multiple of 8
   AXB_D void flush(uint2 *__restrict__ cand, uint32_t row_at, int c0) const
   {
@@ -885,7 +883,7 @@ struct CandStage
 #pragma unroll
     for (int j = 0; j < KNN_STAGE / 2; ++j)
     {
-      const uint2 a = st[(2 * j) * 256 + lane], b = st[(2 * j + 1) * 256 + lane];
+      const uint2 a = st[(2 * j) * STRIDE + lane], b = st[(2 * j + 1) * STRIDE + lane];
       dst[j] = make_uint4(a.x, a.y, b.x, b.y);
     }
   }
@@ -894,14 +892,15 @@ struct CandStage
   {
     const int c0 = c & ~(KNN_STAGE - 1);
     for (int j = 0; j < (c & (KNN_STAGE - 1)); ++j)
-      st[j * 256 + lane] = cand[row_at + c0 + j];
+      st[j * STRIDE + lane] = cand[row_at + c0 + j];
   }
 };
 
-template <int F, int G>
+template <int F, int G, int STRIDE>
 AXB_D int knn_collect_walk(const TreeView &tv, float qx, float qy, float qz, float &R,
                            float &R_hi, float R_lo, float shrink, uint2 *__restrict__ cand,
-                           uint32_t row_at, int cap, CandStage &stage, uint32_t &v_int,
+                           uint32_t row_at, int cap, CandStage<STRIDE> &stage,
+                           uint32_t &v_int,
                            uint32_t &v_leaf)
 {
   constexpr uint32_t SL = leaf_slots<G>(), SI = internal_slots<F>();
@@ -1057,42 +1056,24 @@ AXB_D int knn_collect_walk(const TreeView &tv, float qx, float qy, float qz, flo
 // walk then fits the 64 registers of full occupancy without spilling.
 constexpr int KNN_ROUNDS = 6;
 
-template <int F, int G, int K, bool COUNT>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu((K <= 16 && G == GEOM_POINTS) ? 8 : 1))) void k_knn_collect(
-    TreeView tv, const float *__restrict__ pts, int64_t t0, int64_t tn, int k, int W,
-    const uint32_t *__restrict__ order, uint2 *__restrict__ cand, int cap, float shrink,
-    int max_rounds, uint32_t *__restrict__ ovf, uint32_t *__restrict__ ovf_n,
-    int32_t *__restrict__ oi, float *__restrict__ od, const uint32_t *__restrict__ list,
-    const uint32_t *__restrict__ list_n)
+// Seed and collect walks of one query; returns the entries of its row, or 0
+// when the rounds did not resolve it.
+template <int F, int G, int K, int STRIDE>
+AXB_D int knn_alone(const TreeView &tv, float qx, float qy, float qz, int k, int m, int W,
+                    uint2 *__restrict__ cand, uint32_t row_at, int cap, float shrink,
+                    int max_rounds, CandStage<STRIDE> &stage, uint2 *seed_stage, int &rounds,
+                    uint32_t &v_int, uint32_t &v_leaf)
 {
-  __shared__ __align__(16) uint2 s_stage[G == GEOM_POINTS ? KNN_STAGE * 256 : 1];
-  const int64_t g = (int64_t)xcd_block(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
-  if (g >= tn || (list && t0 + g >= (int64_t)*list_n))
-    return;
-  CandStage stage{s_stage, (int)threadIdx.x};
-  const int64_t t = list ? (int64_t)list[t0 + g] : t0 + g;
-  const int64_t q = order ? (int64_t)order[t] : t;
-  const float qx = pts[3 * q], qy = pts[3 * q + 1], qz = pts[3 * q + 2];
-  const int m = k < tv.n ? k : tv.n;
-  uint32_t v_int = 0, v_leaf = 0;
-  float R = knn_seed<F, G, K>(tv, qx, qy, qz, k, W, v_int, v_leaf,
-                             G == GEOM_POINTS ? s_stage : nullptr);
-  const uint32_t row_at = (uint32_t)(g * cap); // batch * cap + cap <= 2^32 - 1
-  int c = 0;
-  bool done = false;
-  int rounds = 0;
+  float R = knn_seed<F, G, K>(tv, qx, qy, qz, k, W, v_int, v_leaf, seed_stage);
   float R_hi = R;   // radius known to hold >= k points
   float R_lo = 0.f; // radius known to hold < k points
   for (int round = 0; round < max_rounds; ++round)
   {
     ++rounds;
-    c = knn_collect_walk<F, G>(tv, qx, qy, qz, R, R_hi, R_lo, shrink, cand, row_at, cap, stage,
-                               v_int, v_leaf);
+    const int c = knn_collect_walk<F, G>(tv, qx, qy, qz, R, R_hi, R_lo, shrink, cand, row_at,
+                                         cap, stage, v_int, v_leaf);
     if (c >= m && c <= cap)
-    {
-      done = true;
-      break;
-    }
+      return c;
     if (c < m)
     {
       R_lo = R;
@@ -1108,7 +1089,32 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu((K <= 16 &&
       R = next > R_lo ? next : 0.5f * (R_lo + R_hi);
     }
   }
-  if (done) // exact top-k of the row (every leaf within the k-th distance is in it)
+  return 0;
+}
+
+template <int F, int G, int K, bool COUNT>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu((K <= 16 && G == GEOM_POINTS) ? 8 : 1))) void k_knn_collect(
+    TreeView tv, const float *__restrict__ pts, int64_t t0, int64_t tn, int k, int W,
+    const uint32_t *__restrict__ order, uint2 *__restrict__ cand, int cap, float shrink,
+    int max_rounds, uint32_t *__restrict__ ovf, uint32_t *__restrict__ ovf_n,
+    int32_t *__restrict__ oi, float *__restrict__ od)
+{
+  __shared__ __align__(16) uint2 s_stage[G == GEOM_POINTS ? KNN_STAGE * 256 : 1];
+  const int64_t g = (int64_t)xcd_block(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
+  if (g >= tn)
+    return;
+  CandStage<256> stage{s_stage, (int)threadIdx.x};
+  const int64_t t = t0 + g;
+  const int64_t q = order ? (int64_t)order[t] : t;
+  const float qx = pts[3 * q], qy = pts[3 * q + 1], qz = pts[3 * q + 2];
+  const int m = k < tv.n ? k : tv.n;
+  uint32_t v_int = 0, v_leaf = 0;
+  const uint32_t row_at = (uint32_t)(g * cap); // batch * cap + cap <= 2^32 - 1
+  int rounds = 0;
+  const int c = knn_alone<F, G, K>(tv, qx, qy, qz, k, m, W, cand, row_at, cap, shrink,
+                                   max_rounds, stage, G == GEOM_POINTS ? s_stage : nullptr,
+                                   rounds, v_int, v_leaf);
+  if (c > 0) // exact top-k of the row (every leaf within the k-th distance is in it)
     select_row<K>(cand, row_at, c, m, oi, od, q * m);
   else
     ovf[atomicAdd(ovf_n, 1u)] = (uint32_t)t;
@@ -1184,13 +1190,16 @@ AXB_D float group_row_bound(const uint2 *__restrict__ cand, uint32_t row_at, int
 // lane whose row holds between m and cap of them selects its m nearest; the
 // others search again together: a short row with a larger radius, from its
 // count, a full one within its m-th distance.
-// What is left after GROUP_ROUNDS goes to the list for k_knn_collect.
+// Lanes left after GROUP_ROUNDS, or after the first round when they are many
+// (a density that differs a lot within the group), search alone as in
+// k_knn_collect.
 constexpr int GROUP_ROUNDS = 6;
-template <int K, bool COUNT>
+template <int F, int K, bool TOGETHER>
 __global__ __launch_bounds__(256, K <= 16 ? 5 : (K <= 32 ? 4 : 2)) void k_knn_group(
     TreeView tv, const float *__restrict__ pts, int64_t t0, int64_t tn, int k, float want,
-    float spacing, const uint32_t *__restrict__ order, uint2 *__restrict__ cand, int cap,
-    int max_rounds, uint32_t *__restrict__ left, uint32_t *__restrict__ left_n,
+    float spacing, int W, float shrink, const uint32_t *__restrict__ order,
+    uint2 *__restrict__ cand, int cap,
+    int max_rounds, uint32_t *__restrict__ ovf, uint32_t *__restrict__ ovf_n,
     int32_t *__restrict__ oi, float *__restrict__ od)
 {
   __shared__ GroupLds s_group[4];
@@ -1211,19 +1220,23 @@ __global__ __launch_bounds__(256, K <= 16 ? 5 : (K <= 32 ? 4 : 2)) void k_knn_gr
   GroupCand row{cand, real ? (uint32_t)(g * cap) : 0u, cap, 0, make_uint2(0u, 0u)};
   int c = 0, rounds = 0;
   float r = 0.f;
-  if (max_rounds > 0 &&
-      group_guess_radius(tv, L, x, y, z, pending, want, spacing, r, v_int, v_leaf))
+  const int lane = threadIdx.x & 63;
+  bool guessed = max_rounds > 0 && __ballot(pending) != 0;
+  if (guessed)
+    guessed = TOGETHER ? group_guess_radius(tv, L, x, y, z, pending, want, spacing, r, v_int,
+                                            v_leaf)
+                       : group_guess_own_radius(tv, L, x, y, z, pending, want, spacing, r, v_int);
+  if (guessed)
   {
 #pragma unroll 1
     for (int round = 0; round < (max_rounds < GROUP_ROUNDS ? max_rounds : GROUP_ROUNDS); ++round)
     {
-      if (__ballot(pending) == 0)
-        break;
       ++rounds;
       row.cnt = 0;
       if (!group_walk<false>(tv, L, x, y, z, r, sqrt_threshold(r), pending, -1, row, v_int,
                              v_leaf))
         break;
+      wave_lds_order();
       if (pending)
       {
         if (row.cnt >= m && row.cnt <= cap)
@@ -1233,13 +1246,11 @@ __global__ __launch_bounds__(256, K <= 16 ? 5 : (K <= 32 ? 4 : 2)) void k_knn_gr
           pending = false;
         }
         else if (row.cnt < m)
-        {
-          const float f = __builtin_amdgcn_exp2f(
-              (1.f / 3.f) *
-              __builtin_amdgcn_logf(want / (float)(row.cnt > 0 ? row.cnt : 1)));
-          r *= fminf(fmaxf(f, 1.26f), 2.5f);
-        }
+          r *= fminf(fmaxf(approx_cbrt(want / (float)(row.cnt > 0 ? row.cnt : 1)), 1.26f), 2.5f);
       }
+      const uint64_t open = __ballot(pending);
+      if (open == 0 || (!TOGETHER && __popcll(open) > 12))
+        break;
       if (__ballot(pending && row.cnt > cap))
       {
         const float bound = group_row_bound<K>(cand, row.row_at, cap, m);
@@ -1248,13 +1259,21 @@ __global__ __launch_bounds__(256, K <= 16 ? 5 : (K <= 32 ? 4 : 2)) void k_knn_gr
       }
     }
   }
+  wave_lds_order();
+  if (real && c == 0)
+  {
+    CandStage<64> stage{reinterpret_cast<uint2 *>(L.leaf), lane};
+    static_assert(sizeof(L.leaf) >= 64 * KNN_STAGE * sizeof(uint2), "stage of a wavefront");
+    c = knn_alone<F, GEOM_POINTS, K>(tv, x, y, z, k, m, W, cand, row.row_at, cap, shrink,
+                                     max_rounds, stage, nullptr, rounds, v_int, v_leaf);
+  }
   if (c > 0) // exact top-m of the row (every leaf within the m-th distance is in it)
     select_row<K>(cand, row.row_at, c, m, oi, od, q * m);
   else if (real)
-    left[atomicAdd(left_n, 1u)] = (uint32_t)t;
-  if (COUNT && tv.visits && real)
+    ovf[atomicAdd(ovf_n, 1u)] = (uint32_t)t;
+  if (tv.visits && real)
   {
-    atomicAdd(tv.visits + 0, c > 0 ? 1ull : 0ull); // the others are counted by k_knn_collect
+    atomicAdd(tv.visits + 0, 1ull);
     atomicAdd(tv.visits + 1, (unsigned long long)v_int);
     atomicAdd(tv.visits + 2, (unsigned long long)v_leaf);
     atomicAdd(tv.visits + 3, (unsigned long long)c);
@@ -1714,11 +1733,21 @@ int knn_row_capacity(int k, int n) { return knn_shape(k, n).cap; }
 // Leaves the group search aims at for k nearest: a count that is Poisson
 // around k + 4 sqrt(k) + 4 falls below k once in ~10^4.
 static float knn_group_want(int k) { return (float)k + 4.f * std::sqrt((float)k) + 4.f; }
+// Up to this many queries a launch is as long as its slowest wavefronts: a
+// group then goes on together until its last lane is done, from the group's
+// density.  With more, lanes take their own density, and when more than a
+// few of them need another round they walk alone, which costs less work
+// (clustered points, k = 10: 100k queries 0.29 ms together, 0.57 alone; 4M
+// queries 4.6 ms together, 3.3 alone; uniform 0.10 / 0.13 and 1.6 / 1.7).
+constexpr int64_t KNN_TOGETHER_MAX = 300000;
 // Queries of a point tree that are sorted along the Hilbert curve search in
-// groups when they are not far fewer than the points.
+// groups when they are not fewer than half the points (a group of sparser
+// ones sees too many leaves: 1M clustered points, 130k queries, k = 10 0.61
+// -> 0.83 ms), for k >= 2 (the nearest one of 4M uniform points: 0.90 ms
+// alone, 1.03 in groups).
 bool knn_group_rule(const TreeView &tv, int64_t nq, int k)
 {
-  return tv.leaves && k >= 1 && k <= 64 && nq * 8 >= tv.n &&
+  return tv.leaves && k >= 2 && k <= 64 && nq * 2 >= tv.n &&
          (float)tv.n >= 8.f * knn_group_want(k);
 }
 
@@ -1730,46 +1759,43 @@ static hipError_t knn_run(const TreeView &tv, const float *pts, int64_t nq, int 
   const KnnShape sh = knn_shape(k, tv.n);
   const int lim = debug_limits().knn_rounds;
   const int rounds = lim > 0 ? lim : (lim < 0 ? 0 : KNN_ROUNDS);
-  hipError_t e = fill_u32(ws.ovf_n, 0u, 2, s);
-  // points: the group walk first; the list of what it left goes through
-  // the collect launches below
-  const uint32_t *list = nullptr, *list_n = nullptr;
-  if constexpr (G == GEOM_POINTS)
-    if (ws.left)
-    {
-      const float want = knn_group_want(k);
-      float vol = 1.f, longest = 0.f;
-      for (int d = 0; d < 3; ++d)
-        longest = std::max(longest, tv.scene.hi[d] - tv.scene.lo[d]);
-      for (int d = 0; d < 3; ++d)
-        vol *= std::max(tv.scene.hi[d] - tv.scene.lo[d], 1e-3f * longest);
-      const float spacing = std::cbrt(vol / (float)tv.n);
-      for (int64_t t0 = 0; e == hipSuccess && t0 < nq; t0 += ws.batch)
-      {
-        const int64_t tn = std::min(ws.batch, nq - t0);
-        if (tv.visits)
-          AXB_LAUNCH((k_knn_group<K, true>), dim3(grid_of(tn)), dim3(256), 0, s, tv, pts, t0, tn,
-                     k, want, spacing, order, ws.cand, sh.cap, rounds, ws.left, ws.ovf_n + 1, oi,
-                     od);
-        else
-          AXB_LAUNCH((k_knn_group<K, false>), dim3(grid_of(tn)), dim3(256), 0, s, tv, pts, t0,
-                     tn, k, want, spacing, order, ws.cand, sh.cap, rounds, ws.left, ws.ovf_n + 1,
-                     oi, od);
-        e = hipGetLastError();
-      }
-      list = ws.left, list_n = ws.ovf_n + 1;
-    }
+  hipError_t e = fill_u32(ws.ovf_n, 0u, 1, s);
+  // the group search's target and the leaves' spacing
+  const float want = knn_group_want(k);
+  float vol = 1.f, longest = 0.f;
+  for (int d = 0; d < 3; ++d)
+    longest = std::max(longest, tv.scene.hi[d] - tv.scene.lo[d]);
+  for (int d = 0; d < 3; ++d)
+    vol *= std::max(tv.scene.hi[d] - tv.scene.lo[d], 1e-3f * longest);
+  const float spacing = std::cbrt(vol / (float)tv.n);
+  const float per_query = (float)tv.n / (float)nq;
+  const bool together = nq <= KNN_TOGETHER_MAX;
   for (int64_t t0 = 0; e == hipSuccess && t0 < nq; t0 += ws.batch)
   {
     const int64_t tn = std::min(ws.batch, nq - t0);
-    if (tv.visits)
+    bool group = false;
+    if constexpr (G == GEOM_POINTS)
+    {
+      group = order && knn_group_rule(tv, nq, k);
+      if (group && together)
+        AXB_LAUNCH((k_knn_group<F, K, true>), dim3(grid_of(tn)), dim3(256), 0, s, tv, pts, t0,
+                   tn, k, want, spacing, sh.W, sh.shrink, order, ws.cand, sh.cap, rounds, ws.ovf,
+                   ws.ovf_n, oi, od);
+      else if (group)
+        AXB_LAUNCH((k_knn_group<F, K, false>), dim3(grid_of(tn)), dim3(256), 0, s, tv, pts, t0,
+                   tn, k, want, per_query, sh.W, sh.shrink, order, ws.cand, sh.cap, rounds,
+                   ws.ovf, ws.ovf_n, oi, od);
+    }
+    if (group)
+      ;
+    else if (tv.visits)
       AXB_LAUNCH((k_knn_collect<F, G, K, true>), dim3(grid_of(tn)), dim3(256), 0, s, tv, pts, t0,
-                 tn, k, sh.W, order, ws.cand, sh.cap, sh.shrink, rounds, ws.ovf, ws.ovf_n, oi, od,
-                 list, list_n);
+                 tn, k, sh.W, order, ws.cand, sh.cap, sh.shrink, rounds, ws.ovf, ws.ovf_n, oi,
+                 od);
     else
       AXB_LAUNCH((k_knn_collect<F, G, K, false>), dim3(grid_of(tn)), dim3(256), 0, s, tv, pts,
                  t0, tn, k, sh.W, order, ws.cand, sh.cap, sh.shrink, rounds, ws.ovf, ws.ovf_n, oi,
-                 od, list, list_n);
+                 od);
     e = hipGetLastError();
   }
   // unresolved queries of every batch, in one launch at the end: each of
@@ -1809,17 +1835,12 @@ static hipError_t knn_pipeline(const TreeView &tv, const float *pts, int64_t nq,
     batch = (batch + 1) / 2;
   }
   KnnScratch ws{(uint2 *)rows.p, batch, (uint32_t *)dalloc((size_t)nq * sizeof(uint32_t), s),
-                (uint32_t *)dalloc(2 * sizeof(uint32_t), s), nullptr};
-  const bool group = G == GEOM_POINTS && order && knn_group_rule(tv, nq, k);
-  if (group)
-    ws.left = (uint32_t *)dalloc((size_t)nq * sizeof(uint32_t), s);
-  hipError_t e = (ws.cand && ws.ovf && ws.ovf_n && (!group || ws.left)) ? hipSuccess
-                                                                        : hipErrorOutOfMemory;
+                (uint32_t *)dalloc(sizeof(uint32_t), s)};
+  hipError_t e = (ws.cand && ws.ovf && ws.ovf_n) ? hipSuccess : hipErrorOutOfMemory;
   if (e == hipSuccess)
     e = knn_run<F, G, K>(tv, pts, nq, k, order, oi, od, ws, s);
   dfree(ws.ovf, s);
   dfree(ws.ovf_n, s);
-  dfree(ws.left, s);
   return e;
 }
 
