@@ -419,6 +419,7 @@ struct RayPred
 {
   float o[3];
   float d[3];
+  float inv[3]; // 1 / d for the node tests (see ray_node_entry)
 };
 
 // A direction component equal to zero is taken as +0: the slab rule below
@@ -432,6 +433,8 @@ AXB_HD RayPred ray_pred(const float *p6)
   {
     r.o[a] = p6[a];
     r.d[a] = p6[3 + a] == 0.f ? 0.f : p6[3 + a];
+    const float i = 1.f / r.d[a];
+    r.inv[a] = r.d[a] != 0.f && !(fabsf(i) < INFINITY) ? NAN : i;
   }
   return r;
 }
@@ -481,6 +484,31 @@ AXB_HD bool ray_hits(const RayPred &r, const Box6 &b)
   return ray_interval(r, b, t0, t1) && t1 >= 0.f;
 }
 
+// Node boxes: whether the ray may meet box b, and a lower bound of the
+// parameter at which it enters it.  The exact test divides (face - origin)
+// by the direction, six IEEE divisions of ~12 instructions each; here each
+// is a product with 1 / d, off by less than 2^-22 of itself (2^-149 where it
+// is denormal), and the slack below covers both ends.  A component of zero
+// gives infinities with the sign the exact rule has, and 0 * inf = NaN for an
+// origin on a face; NaN -- also that of a component whose reciprocal
+// overflows -- drops out of the min / max, which only widens the interval.
+// (Faces are chosen by the sign of d, not by min / max of the two products,
+// so that a NaN never hides the other face.)  So every box that ray_hits
+// accepts passes, with an entry no larger than ray_distance.
+AXB_HD bool ray_node_entry(const RayPred &r, const Box6 &b, float &entry)
+{
+  float t0 = -INFINITY, t1 = INFINITY;
+#pragma unroll
+  for (int a = 0; a < 3; ++a)
+  {
+    const bool back = r.d[a] < 0.f;
+    t0 = fmaxf(t0, ((back ? b.hi[a] : b.lo[a]) - r.o[a]) * r.inv[a]);
+    t1 = fminf(t1, ((back ? b.lo[a] : b.hi[a]) - r.o[a]) * r.inv[a]);
+  }
+  entry = __builtin_fmaf(t0, 0x1.ffffep-1f, -1e-37f);
+  return t1 >= 0.f && entry <= t1;
+}
+
 // distance(ray, box): the first parameter t >= 0 at which the ray is in the
 // box, +inf if it never is (ArborX_Ray.hpp:429-444); -0 is returned as +0.
 // A box containing another gets a distance no larger (the slab parameters
@@ -509,7 +537,7 @@ AXB_HD SpatialPred sphere_pred(float x, float y, float z, float r)
   SpatialPred p;
   p.cx = x, p.cy = y, p.cz = z, p.thr = sqrt_threshold(r);
   p.qb = Box6{{0.f, 0.f, 0.f}, {0.f, 0.f, 0.f}};
-  p.ray = RayPred{{0.f, 0.f, 0.f}, {0.f, 0.f, 0.f}};
+  p.ray = RayPred{};
   return p;
 }
 AXB_HD SpatialPred box_pred(const Box6 &b)
@@ -517,7 +545,7 @@ AXB_HD SpatialPred box_pred(const Box6 &b)
   SpatialPred p;
   p.cx = p.cy = p.cz = p.thr = 0.f;
   p.qb = b;
-  p.ray = RayPred{{0.f, 0.f, 0.f}, {0.f, 0.f, 0.f}};
+  p.ray = RayPred{};
   return p;
 }
 // p6 = {origin, direction}
@@ -716,8 +744,9 @@ AXB_HD void rope_walk_boxes(const TV &tv, const SpatialPred &pr, uint32_t p, uin
       bx.hi[2] = leaf ? bits_f(s1.z) : bx.hi[2];
     }
     bool pass;
+    float entry;
     if (PK == PRED_RAYS)
-      pass = ray_hits(pr.ray, bx);
+      pass = ray_node_entry(pr.ray, bx, entry); // a leaf is tested exactly below
     else if (PK == PRED_BOXES)
       pass = intersects_bb(pr.qb, bx);
     else
@@ -725,7 +754,8 @@ AXB_HD void rope_walk_boxes(const TV &tv, const SpatialPred &pr, uint32_t p, uin
                   : dist2_pnode(pr.cx, pr.cy, pr.cz, bx) <= pr.thr;
     v_leaf += leaf;
     v_int += !leaf;
-    if (leaf && pass && p != skip && !sink.hit(SLOTS ? (int32_t)p : ~w))
+    if (leaf && pass && p != skip && (PK != PRED_RAYS || ray_hits(pr.ray, bx)) &&
+        !sink.hit(SLOTS ? (int32_t)p : ~w))
       return;
     walk_frame_next<F>(tv, !leaf && pass, bx, fr);
     step = leaf ? SL : (pass ? SI : (uint32_t)w);
@@ -796,6 +826,17 @@ AXB_HD float ordered_distance(const OrderedGeom &g, const Box6 &b)
   return g.kind == PRED_SPHERES ? kmax(dc - g.q[3], 0.f) : dc;
 }
 AXB_HD float ordered_distance(const RayPred &r, const Box6 &b) { return ray_distance(r, b); }
+// A lower bound of the distances of what a node's box holds (+inf: nothing
+// to find there).
+AXB_HD float ordered_node_distance(const OrderedGeom &g, const Box6 &b)
+{
+  return ordered_distance(g, b);
+}
+AXB_HD float ordered_node_distance(const RayPred &r, const Box6 &b)
+{
+  float t;
+  return ray_node_entry(r, b, t) ? kmax(t, 0.f) : INFINITY;
+}
 
 // ------------------------------------------------------- best-first heap
 // Binary min-heap of (key, payload) pairs in private arrays, for the
@@ -921,7 +962,7 @@ AXB_HD bool ordered_walk(const TV &tv, const P &ray, Sink &sink, uint32_t &v_int
   Box6 cb;
   node_box<F>(tv, r0, r1, false, tv.scene, tv.ss, cb);
   ++v_int;
-  if (!(ordered_distance(ray, cb) < INFINITY))
+  if (!(ordered_node_distance(ray, cb) < INFINITY))
     return true;
   bool have_box = true;
   while (true)
@@ -984,7 +1025,7 @@ AXB_HD bool ordered_walk(const TV &tv, const P &ray, Sink &sink, uint32_t &v_int
       ++v_int;
       Box6 nb;
       node_box<F>(tv, a0, F == NODES_FP32 ? tv.slots[q + 1] : a0, left, frame, fs, nb);
-      const float d = ordered_distance(ray, nb);
+      const float d = ordered_node_distance(ray, nb);
       if (d < INFINITY)
         offer(ordered_key(d, 0u), (uint64_t)q | ((uint64_t)(left ? anchor : q) << 32), true, nb);
     };
