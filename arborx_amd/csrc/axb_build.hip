@@ -104,8 +104,9 @@ template <int G>
 __global__ __launch_bounds__(256) void k_morton_hist(
     const float *__restrict__ values, int64_t n,
     const float *__restrict__ scene, uint64_t *__restrict__ keys,
-    uint32_t *__restrict__ hist)
+    uint32_t *__restrict__ hist, int shift0)
 {
+  // digits from bit shift0 on: 8 of them, or 4 from bit 31
   __shared__ uint32_t s_h[8 * 256];
   for (int j = threadIdx.x; j < 8 * 256; j += blockDim.x)
     s_h[j] = 0;
@@ -133,7 +134,8 @@ __global__ __launch_bounds__(256) void k_morton_hist(
     keys[i] = k;
 #pragma unroll
     for (int p = 0; p < 8; ++p)
-      atomicAdd(&s_h[p * 256 + (uint32_t)((k >> (8 * p)) & 255)], 1u);
+      if (p < 4 || shift0 == 0)
+        atomicAdd(&s_h[p * 256 + (uint32_t)((k >> (shift0 + 8 * p)) & 255)], 1u);
   }
   __syncthreads();
   for (int j = threadIdx.x; j < 8 * 256; j += blockDim.x)
@@ -888,7 +890,7 @@ hipError_t build_tree(const float *values, int64_t n, int geometry,
   uint64_t *keys1 = (uint64_t *)dalloc(n * sizeof(uint64_t), stream);
   uint32_t *vals0 = (uint32_t *)dalloc(n * sizeof(uint32_t), stream);
   uint32_t *vals1 = (uint32_t *)dalloc(n * sizeof(uint32_t), stream);
-  uint32_t *hist = (uint32_t *)dalloc(8 * 256 * sizeof(uint32_t), stream);
+  uint32_t *hist = (uint32_t *)dalloc((8 * 256 + SORT_RUN_WORDS) * sizeof(uint32_t), stream);
   float *partials = (float *)dalloc(partial_blocks * 6 * sizeof(float), stream);
   void *ws = dalloc(std::max(sort_ws, scan_ws), stream);
   int32_t *ranges = (int32_t *)dalloc(nint * sizeof(int32_t), stream);
@@ -935,15 +937,15 @@ hipError_t build_tree(const float *values, int64_t n, int geometry,
     const unsigned g = (unsigned)std::min<int64_t>(2048, div_up(n, 256));
     if (geometry == GEOM_POINTS)
       AXB_LAUNCH(k_morton_hist<GEOM_POINTS>, dim3(g), dim3(256), 0, stream, values,
-                         n, out.scene, keys0, hist);
+                         n, out.scene, keys0, hist, sort_hist_shift(n));
     else
       AXB_LAUNCH(k_morton_hist<GEOM_BOXES>, dim3(g), dim3(256), 0, stream, values,
-                         n, out.scene, keys0, hist);
+                         n, out.scene, keys0, hist, sort_hist_shift(n));
   }
 
-  // ---- sort (8 passes of 8 bits; result back in keys0 / vals0)
+  // ---- sort (result back in keys0 / vals0)
   phase.next("ArborX::BVH::BVH::sort_linearized_order");
-  hipError_t e = radix_sort_pairs_u64(keys0, keys1, vals0, vals1, n, 8, hist, ws, err, stream);
+  hipError_t e = sort_keys63(keys0, keys1, vals0, vals1, n, hist, ws, hist + 8 * 256, err, stream);
   if (e != hipSuccess)
     return e;
 

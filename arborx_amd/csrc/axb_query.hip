@@ -1420,7 +1420,7 @@ AXB_D float group_row_bound(const uint2 *__restrict__ cand, uint32_t row_at, int
 // k_knn_collect.
 constexpr int GROUP_ROUNDS = 6;
 template <int F, int K, bool TOGETHER>
-__global__ __launch_bounds__(256, K <= 16 ? 5 : (K <= 32 ? 4 : 2)) void k_knn_group(
+__global__ __launch_bounds__(256, K <= 16 ? 5 : (K <= 32 ? 4 : 2)) void k_knn_collect_group(
     TreeView tv, const float *__restrict__ pts, int64_t t0, int64_t tn, int k, float want,
     float spacing, int W, float shrink, const uint32_t *__restrict__ order,
     uint2 *__restrict__ cand, int cap,
@@ -2003,11 +2003,11 @@ static hipError_t knn_run(const TreeView &tv, const float *pts, int64_t nq, int 
     {
       group = order && knn_group_rule(tv, nq, k);
       if (group && together)
-        AXB_LAUNCH((k_knn_group<F, K, true>), dim3(grid_of(tn)), dim3(256), 0, s, tv, pts, t0,
+        AXB_LAUNCH((k_knn_collect_group<F, K, true>), dim3(grid_of(tn)), dim3(256), 0, s, tv, pts, t0,
                    tn, k, want, spacing, sh.W, sh.shrink, order, ws.cand, sh.cap, rounds, ws.ovf,
                    ws.ovf_n, oi, od);
       else if (group)
-        AXB_LAUNCH((k_knn_group<F, K, false>), dim3(grid_of(tn)), dim3(256), 0, s, tv, pts, t0,
+        AXB_LAUNCH((k_knn_collect_group<F, K, false>), dim3(grid_of(tn)), dim3(256), 0, s, tv, pts, t0,
                    tn, k, want, per_query, sh.W, sh.shrink, order, ws.cand, sh.cap, rounds,
                    ws.ovf, ws.ovf_n, oi, od);
     }
