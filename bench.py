@@ -556,7 +556,10 @@ def main():
         # algorithmic bytes of the traversal kernels, from the node records
         # the kernels themselves count in an untimed pass
         bvh = ax.BoundingVolumeHierarchy(p, node_format=fmt)
-        s_int = 16 if fmt == "q16" else 32
+        # (searches in groups read 32-byte boxes over leaf blocks, whatever
+        # the node format)
+        groups = any("_group" in k for k in kernels)
+        s_int = 16 if fmt == "q16" and not groups else 32
         with ax.profile(timing=False, visits=True) as pv:
             bvh.query(ax.make_intersects(p, r))
         vr = pv.visits
