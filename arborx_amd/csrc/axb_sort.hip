@@ -505,8 +505,9 @@ hipError_t radix_sort_pairs(K *keys0, K *keys1, uint32_t *vals0,
 // the first of its run lists the run: up to RUN_SHORT keys for a thread, up
 // to RUN_LONG for a block.  A longer one, or one whose first inversion comes
 // after RUN_SHORT keys in order, opens the gate of the full sort.  Runs of
-// equal keys hold no inversions.  Bound by one read of the keys: 10M uniform
-// points 0.08 ms, against 0.56 ms for the four passes saved.
+// equal keys hold no inversions.  Bound by the latency of its
+// loads (waves wait for 90 % of their cycles): 10M uniform points 0.07 ms,
+// 1.1 TB/s, where each of the four passes saved takes 0.12 to 0.15 ms.
 constexpr int HI_SHIFT = 31;
 constexpr int RUN_SHORT = 64;
 constexpr int RUN_LONG = 4096;
