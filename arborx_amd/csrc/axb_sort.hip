@@ -505,9 +505,8 @@ hipError_t radix_sort_pairs(K *keys0, K *keys1, uint32_t *vals0,
 // the first of its run lists the run: up to RUN_SHORT keys for a thread, up
 // to RUN_LONG for a block.  A longer one, or one whose first inversion comes
 // after RUN_SHORT keys in order, opens the gate of the full sort.  Runs of
-// equal keys hold no inversions.  Bound by the latency of its
-// loads (waves wait for 90 % of their cycles): 10M uniform points 0.07 ms,
-// 1.1 TB/s, where each of the four passes saved takes 0.12 to 0.15 ms.
+// equal keys hold no inversions.  k_find_runs takes 0.031 ms for the keys of
+// 10M uniform points, each of the four passes saved 0.12 to 0.15 ms.
 constexpr int HI_SHIFT = 31;
 constexpr int RUN_SHORT = 64;
 constexpr int RUN_LONG = 4096;
@@ -555,10 +554,16 @@ AXB_D bool run_at(const uint64_t *__restrict__ keys, int64_t n, int64_t i, int64
 }
 // shorts: starts of the short runs; longs: {start, end} of the long ones.  A
 // block gathers the runs of RUN_TILE keys in LDS and takes its place in the
-// lists with one atomic each (an atomic per run took 0.8 ms for the 41k runs
-// of 5M clustered points).
-constexpr int RUN_TILE = 4096;
-__global__ __launch_bounds__(256) void k_find_runs(const uint64_t *__restrict__ keys, int64_t n,
+// lists with one atomic each.  All of them meet in one word, 20 to 27 ns an
+// atomic, and bound the kernel where most tiles hold a run: one per run took
+// 0.8 ms for the 41k runs of 5M clustered points; one per 4096 keys 0.071 ms
+// for 10M uniform points, one per 16384 keys 0.031 ms (loading 8 steps ahead
+// in tiles of 4096 left it at 0.071 ms).
+constexpr int RUN_TILE = 16384;
+constexpr int RUN_BLOCK = 1024;
+constexpr int RUN_AHEAD = 8;
+static_assert(RUN_TILE % (RUN_BLOCK * RUN_AHEAD) == 0, "whole steps");
+__global__ __launch_bounds__(RUN_BLOCK) void k_find_runs(const uint64_t *__restrict__ keys, int64_t n,
                                                    uint32_t *__restrict__ shorts,
                                                    uint2 *__restrict__ longs, RunWords *w)
 {
@@ -571,17 +576,34 @@ __global__ __launch_bounds__(256) void k_find_runs(const uint64_t *__restrict__ 
   __syncthreads();
   const int64_t base = (int64_t)blockIdx.x * RUN_TILE;
   if (ld_agent(&w->gate) == 0u)
-    for (int j = threadIdx.x; j < RUN_TILE && base + j + 1 < n; j += 256)
+    for (int j = threadIdx.x; j < RUN_TILE && base + j + 1 < n; j += RUN_BLOCK * RUN_AHEAD)
     {
-      int64_t b, e;
-      if (!run_at(keys, n, base + j, b, e))
-        continue;
-      if (e - b <= RUN_SHORT)
-        s_short[atomicAdd(&s_n[0], 1u)] = (uint32_t)b;
-      else if (e - b <= RUN_LONG)
-        s_long[atomicAdd(&s_n[1], 1u)] = make_uint2((uint32_t)b, (uint32_t)e);
-      else
-        st_agent(&w->gate, 1u);
+      uint64_t k[RUN_AHEAD], next[RUN_AHEAD];
+#pragma unroll
+      for (int a = 0; a < RUN_AHEAD; ++a)
+      {
+        const int64_t i = base + j + RUN_BLOCK * a + 1 < n ? base + j + RUN_BLOCK * a : n - 2;
+        k[a] = keys[i];
+        next[a] = keys[i + 1];
+      }
+      uint32_t inversions = 0u;
+#pragma unroll
+      for (int a = 0; a < RUN_AHEAD; ++a)
+        if (base + j + RUN_BLOCK * a + 1 < n && next[a] < k[a] &&
+            (next[a] >> HI_SHIFT) == (k[a] >> HI_SHIFT))
+          inversions |= 1u << a;
+      for (; inversions; inversions &= inversions - 1u)
+      {
+        int64_t b, e;
+        if (!run_at(keys, n, base + j + RUN_BLOCK * (__ffs(inversions) - 1), b, e))
+          continue;
+        if (e - b <= RUN_SHORT)
+          s_short[atomicAdd(&s_n[0], 1u)] = (uint32_t)b;
+        else if (e - b <= RUN_LONG)
+          s_long[atomicAdd(&s_n[1], 1u)] = make_uint2((uint32_t)b, (uint32_t)e);
+        else
+          st_agent(&w->gate, 1u);
+      }
     }
   __syncthreads();
   if (threadIdx.x == 0)
@@ -590,9 +612,9 @@ __global__ __launch_bounds__(256) void k_find_runs(const uint64_t *__restrict__ 
     s_n[3] = s_n[1] ? atomicAdd(&w->longs, s_n[1]) : 0u;
   }
   __syncthreads();
-  for (uint32_t j = threadIdx.x; j < s_n[0]; j += 256)
+  for (uint32_t j = threadIdx.x; j < s_n[0]; j += RUN_BLOCK)
     shorts[s_n[2] + j] = s_short[j];
-  for (uint32_t j = threadIdx.x; j < s_n[1]; j += 256)
+  for (uint32_t j = threadIdx.x; j < s_n[1]; j += RUN_BLOCK)
     longs[s_n[3] + j] = s_long[j];
 }
 
@@ -698,7 +720,7 @@ hipError_t sort_keys63(uint64_t *keys0, uint64_t *keys1, uint32_t *vals0, uint32
   // long one 65)
   RunWords *w = (RunWords *)words;
   uint2 *longs = (uint2 *)keys1;
-  AXB_LAUNCH(k_find_runs, dim3((unsigned)div_up(n, RUN_TILE)), dim3(256), 0, stream, keys0, n, vals1,
+  AXB_LAUNCH(k_find_runs, dim3((unsigned)div_up(n, RUN_TILE)), dim3(RUN_BLOCK), 0, stream, keys0, n, vals1,
              longs, w);
   AXB_LAUNCH(k_fix_runs, dim3(256), dim3(256), 0, stream, keys0, vals0, n, vals1, w);
   AXB_LAUNCH(k_fix_long_runs, dim3(512), dim3(256), 0, stream, keys0, vals0, longs, w);
