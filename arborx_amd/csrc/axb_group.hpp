@@ -136,7 +136,8 @@ AXB_D float group_box_d2(const GroupReach &g, float4 a, float4 b)
 }
 
 // The group's reach.  active: the lane has a finite centre and a radius
-// r >= 0 (thr = sqrt_threshold(r)); other lanes have no hits.  False when
+// r >= 0 (thr = sqrt_threshold(r)); other lanes have no hits (thr is finite
+// or NaN: group_walk leaves infinite ones to the lanes' own walks).  False when
 // the group cannot be searched this way (an infinite radius, or extents at
 // which the halves' error bounds do not hold): every lane then walks alone.
 AXB_D bool group_reach(float x, float y, float z, float r, float thr, bool active,
@@ -371,10 +372,12 @@ AXB_D bool group_walk(const TreeView &tv, GroupLds &L, float x, float y, float z
                       float thr, bool active, int32_t skip, Sink &sink, uint32_t &v_int,
                       uint32_t &v_leaf)
 {
+  // an infinite radius reaches everything, from an infinite (inactive) centre
+  // too
+  if (__ballot(thr == INFINITY || (active && !(thr < INFINITY))))
+    return false;
   if (__ballot(active) == 0)
     return true;
-  if (__ballot(active && !(thr < INFINITY)))
-    return false;
   GroupReach g;
   if (!group_reach(x, y, z, r, thr, active, g))
     return false;

@@ -79,6 +79,23 @@ def test_radii_and_centres_without_hits_or_bounds():
     _check(p, _spheres(p[:600], 0.01), "fp32")
 
 
+@pytest.mark.parametrize("fmt", ["fp32", "q16"])
+@pytest.mark.parametrize("sort", [True, False])
+def test_infinite_radius_at_an_infinite_centre(fmt, sort):
+    # sqrt(inf) <= inf: such a sphere lists every point, whatever the other
+    # predicates of its wavefront are and whether there are any
+    p = synthetic.uniform_points(500, 3)
+    far = np.array([[np.inf, 0, 0, np.inf], [0.5, -np.inf, 0.5, np.inf]], np.float32)
+    s = _spheres(synthetic.uniform_points(640, 4), 0.05)
+    s[[5, 300]] = far  # among ordinary ones
+    assert _check(p, s, fmt, sort) >= 1000
+    assert _check(p, far[:1], fmt, sort) == 500  # alone
+    s[64:128] = far[0]  # a wavefront of them
+    s[130:190, 0] = np.inf  # infinite centres, finite radii
+    s[200] = [np.nan, 0, 0, np.inf]  # no distance at all
+    assert _check(p, s, fmt, sort) >= 66 * 500
+
+
 def test_far_apart_predicates_walk_alone():
     # clusters at the corners of a large cube; wavefronts span several
     g = np.random.default_rng(3)
