@@ -68,7 +68,7 @@ EXPORTED_SYMBOLS = (
     "axb_sqrt_threshold", "axb_morton64_host", "axb_q16_encode_host", "axb_profile_enable",
     "axb_profile_clear",
     "axb_profile_num_records", "axb_profile_record", "axb_profile_visits",
-    "axb_debug_set_limits",
+    "axb_debug_set_limits", "axb_debug_set_memory", "axb_debug_cached_bytes",
 )
 
 
@@ -174,6 +174,8 @@ def lib():
                                           ctypes.POINTER(ctypes.c_double)]),
             "axb_profile_visits": (_I32, [ctypes.POINTER(_I64)]),
             "axb_debug_set_limits": (_I32, [_I64, _I64, _I32]),
+            "axb_debug_set_memory": (_I32, [_I32, _I64]),
+            "axb_debug_cached_bytes": (_I64, []),
         }
         for name, (res, args) in sig.items():
             f = getattr(L, name)
@@ -707,6 +709,32 @@ class debug_limits:
     def __exit__(self, *exc):
         _check(lib().axb_debug_set_limits(0, 0, 0))
         return False
+
+
+class debug_memory:
+    """Test hooks for the device blocks the library keeps between calls
+    (process-wide): scarce makes every allocation fail while blocks are kept,
+    cache_bytes replaces the most that is kept.
+
+    with arborx_amd.debug_memory(cache_bytes=1 << 20):
+        ...
+    """
+
+    def __init__(self, scarce=False, cache_bytes=0):
+        self.args = (1 if scarce else 0, int(cache_bytes))
+
+    def __enter__(self):
+        _check(lib().axb_debug_set_memory(*self.args))
+        return self
+
+    def __exit__(self, *exc):
+        _check(lib().axb_debug_set_memory(0, 0))
+        return False
+
+
+def debug_cached_bytes():
+    """Bytes of device memory kept between calls now."""
+    return lib().axb_debug_cached_bytes()
 
 
 def q16_encode_host(frame6, box6):

@@ -132,13 +132,10 @@ static void keep_pool_memory()
     (void)hipGetLastError();
 }
 
-void *pool_alloc(size_t bytes, hipStream_t stream)
+static void *driver_alloc(size_t bytes, hipStream_t stream)
 {
-  HostScope h("host:pool_alloc");
   keep_pool_memory();
   void *p = nullptr;
-  if (bytes == 0)
-    bytes = 16;
   if (hipMallocAsync(&p, bytes, stream) != hipSuccess)
   {
     (void)hipGetLastError();
@@ -163,11 +160,15 @@ void pool_free(void *p, hipStream_t stream)
 // the stream it was freed on only, so stream order keeps the uses apart as
 // the pool does; the lists hold at most an eighth of the device's memory,
 // what exceeds that goes to the pool, axb_trim_memory returns all of it, and
-// a failing allocation empties the lists before it gives up.
+// an allocation that fails, of whatever kind, empties the lists before it
+// gives up (pool_alloc).
 // hipStreamPerThread is one handle for a stream per thread, so its blocks
 // bypass the cache.
 namespace
 {
+std::atomic<int64_t> g_lim_cache_bytes{0}; // test hooks, see axb_debug_set_memory
+std::atomic<bool> g_lim_scarce{false};
+
 struct CacheKey
 {
   int dev;
@@ -199,6 +200,8 @@ size_t size_class(size_t bytes)
 }
 size_t cache_limit(BlockCache &c, int dev)
 {
+  if (const int64_t lim = g_lim_cache_bytes.load())
+    return (size_t)lim;
   auto it = c.limit.find(dev);
   if (it == c.limit.end())
   {
@@ -226,6 +229,41 @@ static void cache_release_all()
   }
   c.free_blocks.clear();
   c.held.clear();
+}
+
+// Bytes in the lists of all devices.
+static size_t cache_held()
+{
+  BlockCache &c = block_cache();
+  std::lock_guard<std::mutex> lock(c.m);
+  size_t sum = 0;
+  for (auto &kv : c.held)
+    sum += kv.second;
+  return sum;
+}
+
+void *pool_alloc(size_t bytes, hipStream_t stream)
+{
+  HostScope h("host:pool_alloc");
+  if (bytes == 0)
+    bytes = 16;
+  void *p = g_lim_scarce.load() && cache_held() > 0 ? nullptr : driver_alloc(bytes, stream);
+  if (p || cache_held() == 0)
+    return p;
+  // what the cache holds may be what is missing (the device cannot be waited
+  // for while the stream is being captured)
+  hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+  int dev = 0;
+  if (hipStreamIsCapturing(stream, &capture) != hipSuccess ||
+      capture != hipStreamCaptureStatusNone || hipGetDevice(&dev) != hipSuccess ||
+      hipDeviceSynchronize() != hipSuccess)
+  {
+    (void)hipGetLastError();
+    return nullptr;
+  }
+  cache_release_all();
+  (void)hipSetDevice(dev);
+  return driver_alloc(bytes, stream);
 }
 
 void *dalloc(size_t bytes, hipStream_t stream)
@@ -260,20 +298,14 @@ void *dalloc(size_t bytes, hipStream_t stream)
       }
     }
   }
+  size_t got = cls;
   void *p = pool_alloc(cls, stream);
+  if (!p && bytes != 0 && bytes < cls)
+    p = pool_alloc(got = bytes, stream); // not for lack of the class's rest
   if (!p)
-  {
-    // what the cache holds may be what is missing
-    if (hipDeviceSynchronize() != hipSuccess)
-      (void)hipGetLastError();
-    cache_release_all();
-    (void)hipSetDevice(dev);
-    p = pool_alloc(cls, stream);
-    if (!p)
-      return nullptr;
-  }
+    return nullptr;
   std::lock_guard<std::mutex> lock(c.m);
-  c.live[p] = std::make_pair(dev, cls);
+  c.live[p] = std::make_pair(dev, got);
   return p;
 }
 
@@ -606,6 +638,17 @@ axb_status axb_debug_set_limits(int64_t knn_batch_max, int64_t scratch_rows_byte
   g_lim_knn_rounds.store(knn_rounds);
   return AXB_OK;
 }
+
+axb_status axb_debug_set_memory(int32_t scarce, int64_t cache_bytes)
+{
+  if (cache_bytes < 0)
+    AXB_FAIL(AXB_ERR_INVALID_ARGUMENT, "axb_debug_set_memory: bad limit");
+  g_lim_scarce.store(scarce != 0);
+  g_lim_cache_bytes.store(cache_bytes);
+  return AXB_OK;
+}
+
+int64_t axb_debug_cached_bytes(void) { return (int64_t)cache_held(); }
 
 uint64_t axb_morton64_host(const float p[3], const float scene[6])
 {

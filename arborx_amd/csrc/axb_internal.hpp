@@ -28,6 +28,7 @@ void set_error(const std::string &msg);
 
 // Stream-ordered device allocation: pool_* is hipMallocAsync on `stream`;
 // dalloc/dfree keep freed blocks per (device, stream) for the next call.
+// Either empties those lists when the memory they hold is missing.
 void *pool_alloc(size_t bytes, hipStream_t stream);
 void pool_free(void *p, hipStream_t stream);
 void *dalloc(size_t bytes, hipStream_t stream);

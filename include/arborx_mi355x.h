@@ -442,6 +442,14 @@ axb_status axb_profile_visits(int64_t out_host[12]);
 axb_status axb_debug_set_limits(int64_t knn_batch_max, int64_t scratch_rows_bytes,
                                 int32_t knn_rounds);
 
+/* Test hooks for the device blocks kept between calls (no reference
+ * counterpart): scarce != 0 makes every allocation fail while blocks are
+ * kept, as on a full device; cache_bytes > 0 replaces the most that is kept
+ * (an eighth of the device's memory; 0 restores it).  Process-wide; set it
+ * between calls.  axb_debug_cached_bytes: bytes kept now. */
+axb_status axb_debug_set_memory(int32_t scarce, int64_t cache_bytes);
+int64_t axb_debug_cached_bytes(void);
+
 /* Host helper used by the query kernels, exported for unit tests: the largest
  * float s with RN(sqrt(s)) <= r, so that `d2 <= t` decides exactly the
  * reference's `sqrt(d2) <= r` (detail/../geometry/algorithms/

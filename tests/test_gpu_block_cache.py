@@ -1,8 +1,10 @@
 """Blocks that the library keeps between calls: trees and queries of changing
 sizes, from several threads on streams of their own, with trees destroyed
 while others are built, give the rows of a run that keeps nothing."""
+import ctypes
 import threading
 
+import numpy as np
 import pytest
 import torch
 
@@ -61,3 +63,62 @@ def test_trim_gives_kept_blocks_back():
     # ... and given back (the runtime keeps up to a few megabytes of its own)
     assert torch.cuda.mem_get_info()[0] > free - (32 << 20)
     assert rows[0].numel() > 0
+
+
+def test_kept_blocks_give_way_to_allocations_that_fail():
+    # every allocation fails while blocks are kept, as on a full device:
+    # trees, scratch rows, candidate rows, results and energies get memory all
+    # the same
+    n = 30000
+    x = torch.from_numpy(synthetic.uniform_points(n, 1)).cuda()
+    r = synthetic.radius_for_neighbours(n, 12)  # as in _rows
+    want = _rows(n, 1, "q16")
+    L = ax.lib()
+
+    def call(fn, *args):
+        assert fn(*args) == 0, L.axb_last_error()
+
+    def kept():  # something in the lists, and no workspace from earlier calls
+        ax.trim_memory()
+        ax.BVH(x[:5000])
+        assert ax.debug_cached_bytes() > 0
+
+    with ax.debug_memory(scarce=True):
+        kept()
+        tree = ax.BVH(x, node_format="q16")
+        kept()
+        i, o = tree.query(ax.make_intersects(x, r))
+        kept()
+        ki, _, kd = tree.query(ax.make_nearest(x, 5), return_distances=True)
+        for a, b in zip((i, o, ki, kd), want):
+            assert torch.equal(a.cpu(), b)
+        kept()
+        off, idx = ax.energy.neighbour_csr(x, r)
+        kept()
+        e = torch.zeros((), dtype=torch.float64, device="cuda")
+        call(L.axb_pair_energy, ax._ptr(x), n, ax._ptr(off), ax._ptr(idx), ctypes.c_float(r),
+             ctypes.c_void_p(e.data_ptr()), None, ax._stream())
+        # results from the library's own allocator (creating a BVH object
+        # sets torch's again), and the per-thread stream (handle 2), whose
+        # blocks are never kept
+        per_thread = ctypes.c_void_p(2)
+        h, ind, nnz = ctypes.c_void_p(), ctypes.c_void_p(), ctypes.c_int64()
+        offsets = torch.empty(n + 1, dtype=torch.int64, device="cuda")
+        kept()
+        torch.cuda.synchronize()
+        call(L.axb_bvh_create, ax._ptr(x), n, ax.GEOMETRY_POINTS, ax.NODES_Q16, 0, per_thread,
+             ctypes.byref(h))
+        for stream in (ax._stream(), per_thread):
+            kept()
+            call(L.axb_set_output_allocator, ax._ALLOC_FN(0), ax._FREE_FN(0), None)
+            try:
+                call(L.axb_bvh_query_intersects_radius, h, ax._ptr(x), n, ctypes.c_float(r),
+                     ax.TraversalPolicy()._c(), ax._ptr(offsets), ctypes.byref(ind),
+                     ctypes.byref(nnz), stream)
+            finally:
+                ax._use_torch_allocator()
+            assert ind.value not in ax._live_outputs  # not torch's memory
+            call(L.axb_free, ind, stream)
+            assert nnz.value == int(want[1][-1])
+        L.axb_bvh_destroy(h)
+    assert np.isfinite(e.item())
