@@ -158,10 +158,10 @@ void pool_free(void *p, hipStream_t stream)
 // take 2.2 ms), and even the small ones take 2-17 us each (0.36 ms of a
 // 0.97 ms build + two queries of 2k points).  A block is handed out again on
 // the stream it was freed on only, so stream order keeps the uses apart as
-// the pool does; the lists hold at most an eighth of the device's memory,
-// what exceeds that goes to the pool, axb_trim_memory returns all of it, and
-// an allocation that fails, of whatever kind, empties the lists before it
-// gives up (pool_alloc).
+// the pool does; the lists hold at most an eighth of the device's memory
+// (beyond it the blocks freed longest ago go back to the pool, see dfree),
+// axb_trim_memory returns all of it, and an allocation that fails, of
+// whatever kind, empties the lists before it gives up (pool_alloc).
 // hipStreamPerThread is one handle for a stream per thread, so its blocks
 // bypass the cache.
 namespace
@@ -175,10 +175,16 @@ struct CacheKey
   hipStream_t s;
   bool operator<(const CacheKey &o) const { return dev < o.dev || (dev == o.dev && s < o.s); }
 };
+struct FreeBlock
+{
+  void *p;
+  uint64_t tick; // BlockCache::ticks when it was freed
+};
 struct BlockCache
 {
   std::mutex m;
-  std::map<CacheKey, std::map<size_t, std::vector<void *>>> free_blocks;
+  uint64_t ticks = 0;
+  std::map<CacheKey, std::map<size_t, std::vector<FreeBlock>>> free_blocks; // oldest first
   std::unordered_map<void *, std::pair<int, size_t>> live; // block -> device, class
   std::map<int, size_t> held;                              // bytes in free_blocks
   std::map<int, size_t> limit;
@@ -224,11 +230,20 @@ static void cache_release_all()
   {
     (void)hipSetDevice(kv.first.dev);
     for (auto &cls : kv.second)
-      for (void *p : cls.second)
-        (void)hipFree(p);
+      for (const FreeBlock &b : cls.second)
+        (void)hipFree(b.p);
   }
   c.free_blocks.clear();
   c.held.clear();
+}
+
+static bool stream_capturing(hipStream_t stream)
+{
+  hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(stream, &capture) == hipSuccess)
+    return capture != hipStreamCaptureStatusNone;
+  (void)hipGetLastError();
+  return true;
 }
 
 // Bytes in the lists of all devices.
@@ -252,10 +267,8 @@ void *pool_alloc(size_t bytes, hipStream_t stream)
     return p;
   // what the cache holds may be what is missing (the device cannot be waited
   // for while the stream is being captured)
-  hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
   int dev = 0;
-  if (hipStreamIsCapturing(stream, &capture) != hipSuccess ||
-      capture != hipStreamCaptureStatusNone || hipGetDevice(&dev) != hipSuccess ||
+  if (stream_capturing(stream) || hipGetDevice(&dev) != hipSuccess ||
       hipDeviceSynchronize() != hipSuccess)
   {
     (void)hipGetLastError();
@@ -288,7 +301,7 @@ void *dalloc(size_t bytes, hipStream_t stream)
       auto b = it->second.lower_bound(cls);
       if (b != it->second.end() && b->first <= cls + cls / 4)
       {
-        void *p = b->second.back();
+        void *p = b->second.back().p;
         c.live[p] = std::make_pair(dev, b->first);
         c.held[dev] -= b->first;
         b->second.pop_back();
@@ -309,30 +322,98 @@ void *dalloc(size_t bytes, hipStream_t stream)
   return p;
 }
 
+// Takes the blocks freed longest ago out of a device's lists until they hold
+// at most `goal` bytes.
+struct TakenBlock
+{
+  uint64_t tick;
+  CacheKey key;
+  size_t cls;
+  void *p;
+};
+static std::vector<TakenBlock> cache_take_oldest(BlockCache &c, int dev, size_t goal)
+{
+  std::vector<TakenBlock> all;
+  for (auto &kv : c.free_blocks)
+    if (kv.first.dev == dev)
+      for (auto &cls : kv.second)
+        for (const FreeBlock &b : cls.second)
+          all.push_back(TakenBlock{b.tick, kv.first, cls.first, b.p});
+  std::sort(all.begin(), all.end(),
+            [](const TakenBlock &a, const TakenBlock &b) { return a.tick < b.tick; });
+  size_t &held = c.held[dev], taken = 0;
+  for (; taken < all.size() && held > goal; ++taken)
+  {
+    const TakenBlock &t = all[taken];
+    auto list = c.free_blocks.find(t.key);
+    auto cls = list->second.find(t.cls);
+    cls->second.erase(cls->second.begin()); // the oldest of its class
+    if (cls->second.empty())
+      list->second.erase(cls);
+    if (list->second.empty())
+      c.free_blocks.erase(list);
+    held -= t.cls;
+  }
+  all.resize(taken);
+  return all;
+}
+
 void dfree(void *p, hipStream_t stream)
 {
   HostScope h("host:dfree");
   if (!p)
     return;
   BlockCache &c = block_cache();
+  std::vector<TakenBlock> old;
+  int dev = 0;
+  bool keep = false;
   {
     std::lock_guard<std::mutex> lock(c.m);
     auto it = c.live.find(p);
     if (it != c.live.end())
     {
-      const int dev = it->second.first;
+      dev = it->second.first;
       const size_t cls = it->second.second;
       c.live.erase(it);
-      size_t &held = c.held[dev];
-      if (stream != hipStreamPerThread && held + cls <= cache_limit(c, dev))
+      const size_t limit = cache_limit(c, dev);
+      keep = stream != hipStreamPerThread && cls <= limit;
+      if (keep)
       {
-        held += cls;
-        c.free_blocks[CacheKey{dev, stream}][cls].push_back(p);
-        return;
+        c.free_blocks[CacheKey{dev, stream}][cls].push_back(FreeBlock{p, ++c.ticks});
+        c.held[dev] += cls;
+        // full: down to three quarters at once, so that a program whose
+        // sizes drift waits for the device (below) once in many calls
+        if (c.held[dev] > limit && !stream_capturing(stream))
+          old = cache_take_oldest(c, dev, limit - limit / 4);
       }
     }
   }
-  pool_free(p, stream);
+  if (!keep)
+    pool_free(p, stream);
+  if (old.empty())
+    return;
+  // Other streams may still use theirs, and may be gone themselves: once the
+  // device is idle all of them can be freed on this one.
+  bool idle = true;
+  for (const TakenBlock &t : old)
+    if (t.key.s != stream)
+    {
+      int now = 0;
+      idle = hipGetDevice(&now) == hipSuccess && hipSetDevice(dev) == hipSuccess &&
+             hipDeviceSynchronize() == hipSuccess;
+      (void)hipSetDevice(now);
+      (void)hipGetLastError();
+      break;
+    }
+  for (const TakenBlock &t : old)
+    if (idle || t.key.s == stream)
+      pool_free(t.p, stream);
+    else
+    {
+      std::lock_guard<std::mutex> lock(c.m);
+      c.free_blocks[t.key][t.cls].push_back(FreeBlock{t.p, ++c.ticks});
+      c.held[dev] += t.cls;
+    }
 }
 
 // Grow-only workspaces per (device, stream, slot) for the large per-call

@@ -122,3 +122,38 @@ def test_kept_blocks_give_way_to_allocations_that_fail():
             assert nnz.value == int(want[1][-1])
         L.axb_bvh_destroy(h)
     assert np.isfinite(e.item())
+
+
+def test_full_lists_let_the_oldest_blocks_go():
+    # sizes that drift through the size classes, and streams that come and
+    # go: the lists stay within their limit and the newest sizes stay in them
+    limit = 8 << 20
+    ax.trim_memory()
+    points = torch.from_numpy(synthetic.uniform_points(60000, 2)).cuda()
+    want = {}
+    for n in range(9000, 60000, 5100):
+        tree = ax.BVH(points[:n], node_format="q16")
+        want[n] = [t.cpu() for t in tree.query(ax.make_nearest(points[:n], 3))]
+        del tree
+    ax.trim_memory()
+    with ax.debug_memory(cache_bytes=limit):
+        for turn in range(2):
+            for n in want:
+                with torch.cuda.stream(torch.cuda.Stream()):
+                    tree = ax.BVH(points[:n], node_format="q16")
+                    got = tree.query(ax.make_nearest(points[:n], 3))
+                    for a, b in zip(got, want[n]):
+                        assert torch.equal(a.cpu(), b), n
+                    del tree
+                assert 0 < ax.debug_cached_bytes() <= limit
+        # small blocks of the default stream are kept although others filled
+        # the lists before
+        for _ in range(3):
+            tree = ax.BVH(points[:700])
+            full = ax.debug_cached_bytes()
+            del tree
+            assert full < ax.debug_cached_bytes() <= limit
+            with ax.profile(timing=True) as p:
+                ax.BVH(points[:700])
+            assert "host:pool_alloc" not in p.kernels and "host:pool_free" not in p.kernels
+    ax.trim_memory()
