@@ -1185,6 +1185,7 @@ static axb_status query_spatial(const axb_bvh *t, int pred_kind, const float *pr
   // and each row is then sorted by (distance, index); the best-first walk
   // is kept for rows cut at `limit` (it stops early)
   const bool sorted_rows = ordered && limit == INT32_MAX;
+  const bool group = spatial_group_rule(tv, pred_kind, nq);
   auto first = [&](int mode, int32_t *out, int32_t B) {
     if (sorted_rows)
       return launch_ray_slots(tv, t->node_format, preds, nq, order, offsets, out, B, mode, s);
@@ -1192,7 +1193,7 @@ static axb_status query_spatial(const axb_bvh *t, int pred_kind, const float *pr
       return launch_ordered(tv, t->node_format, preds, nq, limit, order, offsets, out, B, mode,
                             s);
     return launch_spatial(tv, t->node_format, t->geometry, pred_kind, preds, nq, radius, order,
-                          offsets, out, B, mode, s);
+                          offsets, out, B, mode, group, s);
   };
   // the overflow list holds rows; the fill pass takes them as its order
   auto fill = [&](const uint32_t *list, int64_t n_list, int32_t *out) {
@@ -1203,7 +1204,7 @@ static axb_status query_spatial(const axb_bvh *t, int pred_kind, const float *pr
       return launch_ordered(tv, t->node_format, preds, n_list, limit, list ? list : order,
                             offsets, out, 0, MODE_FILL, s);
     return launch_spatial(tv, t->node_format, t->geometry, pred_kind, preds, n_list, radius,
-                          list ? list : order, offsets, out, 0, MODE_FILL, s);
+                          list ? list : order, offsets, out, 0, MODE_FILL, group, s);
   };
   // Rows of 96: rows that overflow their scratch row are walked again, and
   // row counts have tails -- rays (1M rays over 5M boxes: mean 10, 0.1%

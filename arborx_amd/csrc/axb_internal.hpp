@@ -400,9 +400,12 @@ constexpr int BUILD_STATUS_WORDS = 8;
 hipError_t build_status(const BuildOut &b, int64_t n, uint32_t *status, hipStream_t stream);
 hipError_t export_topology(const INode *inodes, int64_t nint, int32_t *left_child, int32_t *rope,
                            float *boxes, hipStream_t stream);
+// Whether a batch of nq predicates is searched in groups, which its passes are
+// told (group).
+bool spatial_group_rule(const TreeView &tv, int pred_kind, int64_t nq);
 hipError_t launch_spatial(const TreeView &tv, int node_format, int geometry, int pred_kind,
                           const float *preds, int64_t nq, float radius, const uint32_t *order,
-                          int64_t *offsets, int32_t *out, int32_t buffer, int mode,
+                          int64_t *offsets, int32_t *out, int32_t buffer, int mode, bool group,
                           hipStream_t s);
 // Best-first ray queries over a box tree (rays nq x 6 {origin, unit
 // direction}): row q holds the leaves ray q hits in (distance, index) order,

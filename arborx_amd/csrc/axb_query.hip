@@ -1855,12 +1855,15 @@ static hipError_t launch_spatial_fg(const TreeView &tv, const float *preds, int6
 // Spheres against a point tree go to the group walk when the predicates are
 // not far fewer than the points (64 of them must lie close together): 4M
 // points, 8 neighbours each, alone / in groups: 500k queries 0.33 / 0.24 ms
-// (clustered 0.54 / 0.49), 250k 0.18 / 0.19, 125k 0.13 / 0.18.
-// Rows written again (MODE_FILL) come from such a batch and lie in its
-// densest parts.
-static bool group_rule(const TreeView &tv, int64_t nq, int mode)
+// (clustered 0.54 / 0.49), 250k 0.18 / 0.19, 125k 0.13 / 0.18.  Decided once
+// for a batch: the rows of it that are written again (MODE_FILL) lie in its
+// densest parts (1M points, ~950 hits each, every row written again: 17.8 /
+// 5.7 ms), while those of a sparse batch are sparser still (10k queries, 230
+// hits each, of 1M clustered points: 1.69 / 1.93 ms).
+bool spatial_group_rule(const TreeView &tv, int pred_kind, int64_t nq)
 {
-  return tv.leaves && (mode == MODE_FILL || nq * 8 >= tv.n);
+  return tv.leaves && (pred_kind == PRED_SPHERES || pred_kind == PRED_RADIUS) &&
+         nq * 8 >= tv.n;
 }
 
 template <int F, int PK, bool COUNT>
@@ -1899,10 +1902,10 @@ template <int PK>
 static hipError_t launch_spatial_p(const TreeView &tv, int F, int G, const float *preds,
                                    int64_t nq, float radius, const uint32_t *order,
                                    int64_t *offsets, int32_t *out, int32_t buffer, int mode,
-                                   hipStream_t s)
+                                   bool group, hipStream_t s)
 {
   if constexpr (PK != PRED_BOXES)
-    if (G == GEOM_POINTS && group_rule(tv, nq, mode))
+    if (group)
       return launch_group<PK>(tv, F, preds, nq, radius, order, offsets, out, buffer, mode, s);
   if (F == NODES_FP32 && G == GEOM_POINTS)
     return launch_spatial_fg<NODES_FP32, GEOM_POINTS, PK>(tv, preds, nq, radius, order, offsets,
@@ -1919,7 +1922,7 @@ static hipError_t launch_spatial_p(const TreeView &tv, int F, int G, const float
 
 hipError_t launch_spatial(const TreeView &tv, int node_format, int geometry, int pred_kind,
                           const float *preds, int64_t nq, float radius, const uint32_t *order,
-                          int64_t *offsets, int32_t *out, int32_t buffer, int mode,
+                          int64_t *offsets, int32_t *out, int32_t buffer, int mode, bool group,
                           hipStream_t s)
 {
   if (nq <= 0)
@@ -1935,12 +1938,12 @@ hipError_t launch_spatial(const TreeView &tv, int node_format, int geometry, int
   }
   if (pred_kind == PRED_SPHERES)
     return launch_spatial_p<PRED_SPHERES>(tv, node_format, geometry, preds, nq, radius, order,
-                                          offsets, out, buffer, mode, s);
+                                          offsets, out, buffer, mode, group, s);
   if (pred_kind == PRED_BOXES)
     return launch_spatial_p<PRED_BOXES>(tv, node_format, geometry, preds, nq, radius, order,
-                                        offsets, out, buffer, mode, s);
+                                        offsets, out, buffer, mode, group, s);
   return launch_spatial_p<PRED_RADIUS>(tv, node_format, geometry, preds, nq, radius, order,
-                                       offsets, out, buffer, mode, s);
+                                       offsets, out, buffer, mode, group, s);
 }
 
 // Shape of the collect launches for k <= 64 (the candidate-row capacity and

@@ -105,6 +105,17 @@ def test_far_apart_predicates_walk_alone():
     _check(p, _spheres(p[:6000], 30.0)[::40].copy(), sort=False)
 
 
+@pytest.mark.parametrize("nq,grouped", [(100, False), (2499, False), (2500, True)])
+def test_rows_written_again_go_the_way_of_their_batch(nq, grouped):
+    p = synthetic.uniform_points(20000, 12)
+    s = _spheres(p[:nq], synthetic.radius_for_neighbours(20000, 300))
+    with ax.profile(timing=True) as prof:
+        nnz = _check(p, s)
+    assert nnz > 96 * nq  # rows longer than a scratch row
+    kernels = [k for k in prof.kernels if "k_spatial" in k]
+    assert len(kernels) == 2 and all(("k_spatial_group" in k) == grouped for k in kernels)
+
+
 @pytest.mark.parametrize("n", [2, 65, 4097, 30000])
 def test_neighbour_list_leaves_the_point_out(n):
     p = synthetic.uniform_points(n, 8)
