@@ -791,14 +791,70 @@ __global__ void k_export_topology(const INode *inodes, int nint,
       boxes[6 * k + d] = r.lo[d], boxes[6 * k + 3 + d] = r.hi[d];
 }
 
-__global__ void k_build_status(const float *scene, const int32_t *C, int64_t n,
-                               uint32_t *status)
+// The build's summary for the host.  Word 8, point trees: how the leaves
+// fill space, from the 64 leaf-block boxes below each of up to 64 nodes of
+// the block levels.  fill = 64 times the geometric mean of the boxes' volumes
+// over the node's volume: 1 for uniform points, 1/8 on a surface, 1/4096 on a
+// line, small where the density changes a lot within a node.
+constexpr int STATUS_WAVES = 16, STATUS_NODES = 64;
+__global__ __launch_bounds__(64 * STATUS_WAVES) void k_build_status(
+    const float *scene, const int32_t *C, int64_t n, const float4 *__restrict__ blk,
+    uint32_t blocks, uint32_t *status)
 {
-  const int t = threadIdx.x;
+  const int t = threadIdx.x, lane = t & 63;
   if (t == 0)
     status[1] = n > 1 ? (uint32_t)C[n - 1] : 0u;
   else if (t < 7)
     status[1 + t] = f_bits(scene[t - 1]);
+  __shared__ uint32_t s_over[3]; // nodes of a fill of at least 0.1, 0.25, 0.35
+  if (t < 3)
+    s_over[t] = 0u;
+  __syncthreads();
+  const uint32_t nodes = (blocks + 63u) / 64u;
+  const uint32_t looks = nodes < (uint32_t)STATUS_NODES ? nodes : (uint32_t)STATUS_NODES;
+  for (uint32_t j = (uint32_t)t / 64u; j < looks; j += STATUS_WAVES)
+  {
+    // one node of each 1/64 of them, at a different place in each: nodes at
+    // regular distances would all begin at the corners of large octants
+    const uint64_t at = (uint64_t)j * 65536u + ((j * 40503u) & 65535u);
+    const uint32_t node = (uint32_t)(at * nodes / ((uint64_t)looks * 65536u));
+    const uint32_t b = node * 64u + (uint32_t)lane;
+    const uint32_t m = blocks - node * 64u < 64u ? blocks - node * 64u : 64u;
+    float lo[3] = {FLT_MAX, FLT_MAX, FLT_MAX}, hi[3] = {-FLT_MAX, -FLT_MAX, -FLT_MAX};
+    // log2 of a volume; an axis counts for at least 1/1000 of the longest
+    auto log_volume = [](const float (&l)[3], const float (&h)[3]) {
+      const float x = h[0] - l[0], y = h[1] - l[1], z = h[2] - l[2];
+      const float least = fmaxf(1e-3f * fmaxf(fmaxf(x, y), z), 1e-30f);
+      return __log2f(fmaxf(x, least)) + __log2f(fmaxf(y, least)) + __log2f(fmaxf(z, least));
+    };
+    float logs = 0.f;
+    if (b < blocks)
+    {
+      const float4 p = blk[2 * (size_t)b], q = blk[2 * (size_t)b + 1];
+      lo[0] = p.x, lo[1] = p.y, lo[2] = p.z, hi[0] = p.w, hi[1] = q.x, hi[2] = q.y;
+      logs = log_volume(lo, hi);
+    }
+    wave_bounds(lo, hi);
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1)
+      logs += __shfl_xor(logs, o, 64);
+    const float fill = __log2f((float)m) + logs / (float)m - log_volume(lo, hi);
+    if (lane == 0)
+    {
+      if (fill >= -3.3219281f)
+        atomicAdd(&s_over[0], 1u);
+      if (fill >= -2.f)
+        atomicAdd(&s_over[1], 1u);
+      if (fill >= -1.5145732f)
+        atomicAdd(&s_over[2], 1u);
+    }
+  }
+  __syncthreads();
+  if (t == 0)
+    status[8] = 16u * s_over[1] >= 15u * looks ? FILL_UNIFORM
+                : 2u * s_over[2] >= looks      ? FILL_EVEN
+                : 2u * s_over[0] >= looks      ? FILL_UNEVEN
+                                               : FILL_THIN;
 }
 
 inline unsigned grid_for(int64_t n, int block = 256)
@@ -1078,7 +1134,8 @@ hipError_t build_tree(const float *values, int64_t n, int geometry,
 
 hipError_t build_status(const BuildOut &b, int64_t n, uint32_t *status, hipStream_t stream)
 {
-  AXB_LAUNCH(k_build_status, dim3(1), dim3(64), 0, stream, b.scene, b.C, n, status);
+  AXB_LAUNCH(k_build_status, dim3(1), dim3(64 * STATUS_WAVES), 0, stream, b.scene, b.C, n, b.blk,
+             b.blk ? block_levels(n).count[0] : 0u, status);
   return hipGetLastError();
 }
 

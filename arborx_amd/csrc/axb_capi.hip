@@ -550,6 +550,7 @@ struct axb_bvh
   bool keep_topology = false;
   BuildOut b{};
   float bounds[6];
+  int32_t fill = FILL_UNIFORM;
   hipStream_t stream = nullptr;
   uint32_t *d_err = nullptr;
 };
@@ -644,6 +645,7 @@ static TreeView view_of(const axb_bvh *t, uint32_t *err)
   tv.blk = t->b.blk;
   const BlockLevels bl = block_levels(t->n);
   tv.blk_levels = (int32_t)bl.levels;
+  tv.fill = t->fill;
   for (int l = 0; l < BLOCK_LEVELS_MAX; ++l)
     tv.blk_at[l] = bl.at[l], tv.blk_count[l] = bl.count[l];
   for (int d = 0; d < 3; ++d)
@@ -784,6 +786,7 @@ axb_status axb_bvh_create(const float *values, int64_t n, int32_t geometry, int3
     e = sync_stream(s);
   const int32_t c_last = (int32_t)status[1];
   std::memcpy(t->bounds, status + 2, sizeof(t->bounds));
+  t->fill = (int32_t)status[8];
   if (e == hipSuccess && n > 0)
   {
     const int64_t sl = geometry == AXB_GEOMETRY_POINTS ? 1 : 2;

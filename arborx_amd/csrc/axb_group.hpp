@@ -22,7 +22,8 @@
 //   4. each lane tests the candidates in its mask with the exact float
 //      distance, in leaf order: results and their order are the rope walk's.
 // A wavefront whose predicates are not close together (or not finite) finds
-// too many blocks and is sent back to walk the tree lane by lane.
+// too many blocks, or more candidates than pay (group_pays), and is sent back
+// to walk the tree lane by lane.
 #pragma once
 
 #include "axb_internal.hpp"
@@ -80,6 +81,13 @@ AXB_D float wave_max(float v)
     v = fmaxf(v, __shfl_xor(v, o, 64));
   return v;
 }
+AXB_D float wave_sum(float v)
+{
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1)
+    v += __shfl_xor(v, o, 64);
+  return v;
+}
 AXB_D float wave_uniform(float v)
 {
   return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(v)));
@@ -96,7 +104,8 @@ AXB_D uint32_t lanes_below(uint64_t m)
 struct GroupReach
 {
   float lo[3], hi[3], mid[3];
-  float thr, scale;
+  float r, thr, scale;
+  float tiny; // far below any extent that matters
 };
 
 // A candidate's terms of the matrix product: {x y z |p|^2 high} in lanes
@@ -156,6 +165,8 @@ AXB_D bool group_reach(float x, float y, float z, float r, float thr, bool activ
   const float rm = wave_uniform(wave_max(active ? r : 0.f));
   g.thr = wave_uniform(wave_max(active ? thr : 0.f));
   h = h + rm;
+  g.r = rm;
+  g.tiny = 1e-6f * h;
   g.scale = GROUP_EXTENT / h;
   // below 1e-12 squared distances may be denormal, above 1e15 overflow
   return h > 1e-12f && h < 1e15f;
@@ -212,6 +223,49 @@ AXB_D int group_blocks(const TreeView &tv, const GroupReach &g, GroupLds &L, int
   wave_lds_order();
   buffer = cur;
   return cnt;
+}
+
+// The part of a block's box, and so about of its leaves, within the box of
+// the group's reach.
+AXB_D float group_part(const GroupReach &g, float4 a, float4 b)
+{
+  const float bl[3] = {a.x, a.y, a.z}, bh[3] = {a.w, b.x, b.y};
+  float part = 1.f;
+#pragma unroll
+  for (int d = 0; d < 3; ++d)
+  {
+    const float cut = fminf(bh[d], g.hi[d] + g.r) - fmaxf(bl[d], g.lo[d] - g.r);
+    part *= fmaxf(cut, g.tiny) * __builtin_amdgcn_rcpf(fmaxf(bh[d] - bl[d], g.tiny));
+  }
+  return part;
+}
+
+// What the search of a group is compared with: the walks of its 64 lanes take
+// about base + per_hit * hits vector instructions per wavefront.  known: hits
+// of a lane as far as the caller knows them (else 0).
+struct LoneCost
+{
+  float base, per_hit, known;
+};
+
+// Whether searching `leaves` candidates together is less work.  A candidate
+// costs 2.2 instructions for its leaf and mask bit, and up to 15 in the exact
+// loop, which runs as often as the busiest lane has candidates in a window:
+// a lane's hits lie together, so about hits / GROUP_CAND of the time.
+AXB_D bool group_pays(const GroupReach &g, float leaves, float r, bool active,
+                      const LoneCost &lone)
+{
+  // hits of a lane, on average: leaves in its sphere if all are spread over
+  // the box of the reach (volumes in the group's own unit)
+  float box = (float)__popcll(__ballot(active));
+#pragma unroll
+  for (int d = 0; d < 3; ++d)
+    box *= fmaxf(g.hi[d] - g.lo[d] + 2.f * g.r, g.tiny) * g.scale;
+  const float u = active ? r * g.scale : 0.f;
+  const float spheres = wave_uniform(wave_sum(4.18879f * u * u * u));
+  const float hits = fmaxf(lone.known, leaves * spheres * __builtin_amdgcn_rcpf(box));
+  return leaves * (2.2f + 0.094f * fminf(hits, (float)GROUP_CAND)) <=
+         lone.base + lone.per_hit * hits;
 }
 
 // The lane's predicate as the two matrix operands (columns 0-31 and 32-63
@@ -369,8 +423,8 @@ AXB_D void group_leaves(const TreeView &tv, const GroupLds &L, int nodes, int bu
 // reported.
 template <bool SKIP, class Sink>
 AXB_D bool group_walk(const TreeView &tv, GroupLds &L, float x, float y, float z, float r,
-                      float thr, bool active, int32_t skip, Sink &sink, uint32_t &v_int,
-                      uint32_t &v_leaf)
+                      float thr, bool active, int32_t skip, const LoneCost &lone, Sink &sink,
+                      uint32_t &v_int, uint32_t &v_leaf)
 {
   // an infinite radius reaches everything, from an infinite (inactive) centre
   // too
@@ -382,9 +436,13 @@ AXB_D bool group_walk(const TreeView &tv, GroupLds &L, float x, float y, float z
   if (!group_reach(x, y, z, r, thr, active, g))
     return false;
   int buffer = 0;
+  float part = 0.f;
   const int nodes =
-      group_blocks(tv, g, L, buffer, v_int, [](uint64_t, const float4 &, const float4 &) {});
-  if (nodes < 0)
+      group_blocks(tv, g, L, buffer, v_int, [&](uint64_t m, const float4 &a, const float4 &b) {
+        if ((m >> (threadIdx.x & 63)) & 1u)
+          part += group_part(g, a, b);
+      });
+  if (nodes < 0 || !group_pays(g, 64.f * wave_uniform(wave_sum(part)), r, active, lone))
     return false;
   half4_t col[2];
   group_columns(g, x, y, z, r, active, col);

@@ -246,7 +246,13 @@ struct TreeView
   const float4 *blk;          // boxes of BlockLevels
   int32_t blk_levels;
   uint32_t blk_at[BLOCK_LEVELS_MAX], blk_count[BLOCK_LEVELS_MAX];
+  int32_t fill; // FILL_*
 };
+
+// How the leaves of a point tree fill space (k_build_status): on surfaces,
+// curves or in tight clusters, unevenly, evenly in most places, evenly
+// everywhere.
+constexpr int32_t FILL_THIN = 0, FILL_UNEVEN = 1, FILL_EVEN = 2, FILL_UNIFORM = 3;
 
 constexpr int MODE_COUNT = 0;
 constexpr int MODE_FILL = 1;
@@ -395,8 +401,9 @@ hipError_t scene_box(const float *values, int64_t n, int geometry, float *scene,
 hipError_t build_tree(const float *values, int64_t n, int geometry, int node_format,
                       bool keep_topology, uint32_t *err, hipStream_t stream, BuildOut &out);
 // Words of a build's status block: {error word, C[n - 1] (0 when n < 2),
-// scene box (6 floats)}; build_status fills words 1..7 after build_tree.
-constexpr int BUILD_STATUS_WORDS = 8;
+// scene box (6 floats), how a point tree's leaves fill space}; build_status
+// fills words 1..8 after build_tree.
+constexpr int BUILD_STATUS_WORDS = 9;
 hipError_t build_status(const BuildOut &b, int64_t n, uint32_t *status, hipStream_t stream);
 hipError_t export_topology(const INode *inodes, int64_t nint, int32_t *left_child, int32_t *rope,
                            float *boxes, hipStream_t stream);

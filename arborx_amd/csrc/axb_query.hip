@@ -82,6 +82,24 @@ __global__ __launch_bounds__(256) void k_spatial(
   }
 }
 
+// What 64 lanes' rope walks cost (LoneCost), fitted to k_spatial at 4 to 1000
+// hits.  Where the leaves lie on surfaces or curves the walks are cheaper for
+// their hits.  A row that is written again is as long as its offsets say.
+// Measured alone / together with no limit / with this one: 10M points in
+// clusters too tight for the query order (sigma 0.0005) 9.5 / 11.6 / 9.1 ms,
+// 16k unsorted predicates, 30 hits 0.32 / 0.57 / 0.24, 1M points on a line,
+// 32 hits 0.71 / 1.45 / 0.69; uniform 10M unchanged (6.8 / 3.6 / 3.6).
+template <int MODE>
+AXB_D LoneCost rope_walk_cost(const TreeView &tv, const int64_t *__restrict__ offsets, int64_t q,
+                              bool real)
+{
+  const float a = tv.fill == FILL_THIN ? 1.f : 1.6f;
+  LoneCost c{a * 2600.f, a * 400.f, 0.f};
+  if (MODE == MODE_FILL)
+    c.known = wave_uniform(wave_max(real ? (float)(offsets[q + 1] - offsets[q]) : 0.f));
+  return c;
+}
+
 // Spheres against points, 64 lanes searching together (axb_group.hpp).  10M
 // uniform points, ~32 neighbours: 5.31 (k_spatial) -> 2.27 ms, 6650 vector
 // instructions per wavefront, 72% of the issue rate; six wavefronts per SIMD
@@ -115,8 +133,8 @@ __global__ __launch_bounds__(256, 6) void k_spatial_group(
   if (real)
     rw.init(out, offsets, q, buffer);
   uint32_t v_int = 0, v_leaf = 0;
-  if (!group_walk<false>(tv, s_group[threadIdx.x >> 6], x, y, z, r, thr, active, -1, rw, v_int,
-                         v_leaf) &&
+  if (!group_walk<false>(tv, s_group[threadIdx.x >> 6], x, y, z, r, thr, active, -1,
+                         rope_walk_cost<MODE>(tv, offsets, q, real), rw, v_int, v_leaf) &&
       real)
   {
     const SpatialPred pr = sphere_pred(x, y, z, r);
@@ -575,7 +593,7 @@ __global__ __launch_bounds__(256, 6) void k_nlist_group(TreeView tv, float radiu
       real && fabsf(x) < INFINITY && fabsf(y) < INFINITY && fabsf(z) < INFINITY;
   uint32_t v_int = 0, v_leaf = 0;
   if (!group_walk<true>(tv, s_group[threadIdx.x >> 6], x, y, z, radius, thr, active, (int32_t)q,
-                        rw, v_int, v_leaf) &&
+                        rope_walk_cost<MODE>(tv, offsets, q, real), rw, v_int, v_leaf) &&
       real)
   {
     constexpr uint32_t SL = leaf_slots<GEOM_POINTS>(), SI = internal_slots<F>();
@@ -1470,8 +1488,8 @@ __global__ __launch_bounds__(256, K <= 16 ? 5 : (K <= 32 ? 4 : 2)) void k_knn_co
     {
       ++rounds;
       row.cnt = 0;
-      if (!group_walk<false>(tv, L, x, y, z, r, sqrt_threshold(r), pending, -1, row, v_int,
-                             v_leaf))
+      if (!group_walk<false>(tv, L, x, y, z, r, sqrt_threshold(r), pending, -1,
+                             LoneCost{FLT_MAX, 0.f, 0.f}, row, v_int, v_leaf))
         break;
       wave_lds_order();
       if (pending)

@@ -188,3 +188,35 @@ def test_nearest_ties_and_lists_of_queries_left():
             if x.numel() == 6 * len(q):
                 x, y = x.reshape(-1, 6)[keep], y.reshape(-1, 6)[keep]
             assert torch.equal(x, y), kw
+
+
+# ------------------------------------------- what is left to the lanes' walks
+def _leaves_per_query(points, spheres, sort):
+    tree = ax.BVH(torch.from_numpy(points).cuda(), node_format="q16")
+    q = ax.intersects(ax.Spheres(torch.from_numpy(spheres)))
+    with ax.profile(timing=False, visits=True) as prof:
+        tree.query(q, ax.TraversalPolicy(0, sort))
+    _check(points, spheres, sort=sort)
+    return prof.visits["leaf"] / len(spheres)
+
+
+def test_groups_that_do_not_pay_walk_alone():
+    # visits count blocks of 64 leaves for a group's lanes, leaves for a lane
+    # alone: a group over all leaves looks at n / 64 blocks
+    n = 16000
+    g = np.random.default_rng(1)
+    p = synthetic.uniform_points(n, 3)
+    r = synthetic.radius_for_neighbours(n, 30)
+    assert _leaves_per_query(p, _spheres(p[g.permutation(n)], r), False) < 200  # not 250
+    assert _leaves_per_query(p, _spheres(p, r), True) < 40  # close together: groups
+    # on a line every cell of the query order holds thousands of points
+    line = np.full((1 << 20, 3), 0.5, np.float32)
+    line[:, 0] = synthetic.uniform01(7, 1 << 20)
+    assert _leaves_per_query(line, _spheres(line, 8.0 / (1 << 20)), True) < 40  # not 64
+
+
+@pytest.mark.parametrize("scale", [1e-11, 1e-4, 1e8, 1e13])
+def test_cost_of_a_group_at_any_scale(scale):
+    p = (synthetic.uniform_points(20000, 3) * np.float32(scale)).astype(np.float32)
+    r = np.float32(synthetic.radius_for_neighbours(20000, 30) * scale)
+    assert _leaves_per_query(p, _spheres(p, r), True) < 40
