@@ -68,7 +68,8 @@ EXPORTED_SYMBOLS = (
     "axb_sqrt_threshold", "axb_morton64_host", "axb_q16_encode_host", "axb_profile_enable",
     "axb_profile_clear",
     "axb_profile_num_records", "axb_profile_record", "axb_profile_visits",
-    "axb_debug_set_limits", "axb_debug_set_memory", "axb_debug_cached_bytes",
+    "axb_debug_set_limits", "axb_debug_set_search", "axb_debug_set_memory",
+    "axb_debug_cached_bytes",
 )
 
 
@@ -174,6 +175,7 @@ def lib():
                                           ctypes.POINTER(ctypes.c_double)]),
             "axb_profile_visits": (_I32, [ctypes.POINTER(_I64)]),
             "axb_debug_set_limits": (_I32, [_I64, _I64, _I32]),
+            "axb_debug_set_search": (_I32, [_I64, _I32]),
             "axb_debug_set_memory": (_I32, [_I32, _I64]),
             "axb_debug_cached_bytes": (_I64, []),
         }
@@ -708,6 +710,27 @@ class debug_limits:
 
     def __exit__(self, *exc):
         _check(lib().axb_debug_set_limits(0, 0, 0))
+        return False
+
+
+class debug_search:
+    """Replaces what the rules of the searches of 64 lanes together go by
+    (tests only; process-wide): the most nearest queries of a small launch and
+    how the leaves fill space (0 thinly .. 3 uniformly, -1: as measured).
+
+    with arborx_amd.debug_search(knn_small=1, fill=2):
+        ...
+    """
+
+    def __init__(self, knn_small=0, fill=-1):
+        self.args = (int(knn_small), int(fill))
+
+    def __enter__(self):
+        _check(lib().axb_debug_set_search(*self.args))
+        return self
+
+    def __exit__(self, *exc):
+        _check(lib().axb_debug_set_search(0, -1))
         return False
 
 

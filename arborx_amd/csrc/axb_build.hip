@@ -795,7 +795,10 @@ __global__ void k_export_topology(const INode *inodes, int nint,
 // fill space, from the 64 leaf-block boxes below each of up to 64 nodes of
 // the block levels.  fill = 64 times the geometric mean of the boxes' volumes
 // over the node's volume: 1 for uniform points, 1/8 on a surface, 1/4096 on a
-// line, small where the density changes a lot within a node.
+// line, small where the density changes a lot within a node.  Medians of 50k
+// to 4M points: uniform 0.9 to 1.2, normal 0.27 to 0.94, 1000 clusters of
+// sigma 0.01 0.11 to 0.40, a sphere 0.11 to 0.13, a helix below 0.01.  Even:
+// half the nodes above 0.35, uneven: above 0.1, uniform: 7/8 above 0.25.
 constexpr int STATUS_WAVES = 16, STATUS_NODES = 64;
 __global__ __launch_bounds__(64 * STATUS_WAVES) void k_build_status(
     const float *scene, const int32_t *C, int64_t n, const float4 *__restrict__ blk,
@@ -851,10 +854,10 @@ __global__ __launch_bounds__(64 * STATUS_WAVES) void k_build_status(
   }
   __syncthreads();
   if (t == 0)
-    status[8] = 16u * s_over[1] >= 15u * looks ? FILL_UNIFORM
-                : 2u * s_over[2] >= looks      ? FILL_EVEN
-                : 2u * s_over[0] >= looks      ? FILL_UNEVEN
-                                               : FILL_THIN;
+    status[8] = 8u * s_over[1] >= 7u * looks ? FILL_UNIFORM
+                : 2u * s_over[2] >= looks    ? FILL_EVEN
+                : 2u * s_over[0] >= looks    ? FILL_UNEVEN
+                                             : FILL_THIN;
 }
 
 inline unsigned grid_for(int64_t n, int block = 256)

@@ -441,11 +441,14 @@ std::map<WsKey, std::array<WsBlock, WS_NUM>> g_ws;
 std::atomic<int64_t> g_lim_knn_batch{0};
 std::atomic<int64_t> g_lim_rows_bytes{0};
 std::atomic<int32_t> g_lim_knn_rounds{0};
+std::atomic<int64_t> g_lim_knn_small{0};
+std::atomic<int32_t> g_lim_fill{0};
 } // namespace
 
 Limits debug_limits()
 {
-  return Limits{g_lim_knn_batch.load(), g_lim_rows_bytes.load(), g_lim_knn_rounds.load()};
+  return Limits{g_lim_knn_batch.load(), g_lim_rows_bytes.load(), g_lim_knn_rounds.load(),
+                g_lim_knn_small.load(), g_lim_fill.load()};
 }
 
 void WsLease::acquire(hipStream_t s_, int slot_, size_t bytes)
@@ -645,7 +648,8 @@ static TreeView view_of(const axb_bvh *t, uint32_t *err)
   tv.blk = t->b.blk;
   const BlockLevels bl = block_levels(t->n);
   tv.blk_levels = (int32_t)bl.levels;
-  tv.fill = t->fill;
+  const int32_t fill = debug_limits().fill;
+  tv.fill = fill > 0 ? fill - 1 : t->fill;
   for (int l = 0; l < BLOCK_LEVELS_MAX; ++l)
     tv.blk_at[l] = bl.at[l], tv.blk_count[l] = bl.count[l];
   for (int d = 0; d < 3; ++d)
@@ -719,6 +723,15 @@ axb_status axb_debug_set_limits(int64_t knn_batch_max, int64_t scratch_rows_byte
   g_lim_knn_batch.store(knn_batch_max);
   g_lim_rows_bytes.store(scratch_rows_bytes);
   g_lim_knn_rounds.store(knn_rounds);
+  return AXB_OK;
+}
+
+axb_status axb_debug_set_search(int64_t knn_small, int32_t fill)
+{
+  if (knn_small < 0 || fill < -1 || fill > FILL_UNIFORM)
+    AXB_FAIL(AXB_ERR_INVALID_ARGUMENT, "axb_debug_set_search: bad limit");
+  g_lim_knn_small.store(knn_small);
+  g_lim_fill.store(fill + 1);
   return AXB_OK;
 }
 

@@ -240,32 +240,72 @@ AXB_D float group_part(const GroupReach &g, float4 a, float4 b)
   return part;
 }
 
-// What the search of a group is compared with: the walks of its 64 lanes take
-// about base + per_hit * hits vector instructions per wavefront.  known: hits
-// of a lane as far as the caller knows them (else 0).
-struct LoneCost
+// Whether a group's search is less work than the walks of its 64 lanes, by the
+// number of candidates.  A candidate costs 2.2 vector instructions per
+// wavefront for its leaf and mask bit, and up to 15 in the exact loop, which
+// runs as often as the busiest lane has candidates in a window: a lane's hits
+// lie together, so about hits / GROUP_CAND of the time.
+AXB_D float group_cost(float leaves, float hits)
+{
+  return leaves * (2.2f + 0.094f * fminf(hits, (float)GROUP_CAND));
+}
+// Walks that take about base + per_hit * hits instructions (base FLT_MAX: no
+// limit).  known: hits of a lane as far as the caller knows them (else 0).
+struct WalkCost
 {
   float base, per_hit, known;
+  float share; // of the reach's box in a lane's sphere, on average
+  AXB_D void meet(const GroupReach &g, float r, bool active)
+  {
+    if (base == FLT_MAX)
+      return;
+    float box = (float)__popcll(__ballot(active)); // volumes in the group's own unit
+#pragma unroll
+    for (int d = 0; d < 3; ++d)
+      box *= fmaxf(g.hi[d] - g.lo[d] + 2.f * g.r, g.tiny) * g.scale;
+    const float u = active ? r * g.scale : 0.f;
+    share = wave_uniform(wave_sum(4.18879f * u * u * u)) * __builtin_amdgcn_rcpf(box);
+  }
+  AXB_D bool pays(float leaves) const
+  {
+    const float hits = fmaxf(known, leaves * share);
+    return group_cost(leaves, hits) <= base + per_hit * hits;
+  }
+};
+// At most so many candidates.
+struct LeafLimit
+{
+  float most;
+  AXB_D void meet(const GroupReach &, float, bool) {}
+  AXB_D bool pays(float leaves) const { return leaves <= most; }
+};
+struct NoLimit
+{
+  AXB_D void meet(const GroupReach &, float, bool) {}
+  AXB_D bool pays(float) const { return true; }
 };
 
-// Whether searching `leaves` candidates together is less work.  A candidate
-// costs 2.2 instructions for its leaf and mask bit, and up to 15 in the exact
-// loop, which runs as often as the busiest lane has candidates in a window:
-// a lane's hits lie together, so about hits / GROUP_CAND of the time.
-AXB_D bool group_pays(const GroupReach &g, float leaves, float r, bool active,
-                      const LoneCost &lone)
+// Whether searching the blocks that group_blocks found pays.
+template <class Limit>
+AXB_D bool group_pays(const TreeView &tv, const GroupReach &g, const GroupLds &L, int nodes,
+                      int buffer, const Limit &limit)
 {
-  // hits of a lane, on average: leaves in its sphere if all are spread over
-  // the box of the reach (volumes in the group's own unit)
-  float box = (float)__popcll(__ballot(active));
-#pragma unroll
-  for (int d = 0; d < 3; ++d)
-    box *= fmaxf(g.hi[d] - g.lo[d] + 2.f * g.r, g.tiny) * g.scale;
-  const float u = active ? r * g.scale : 0.f;
-  const float spheres = wave_uniform(wave_sum(4.18879f * u * u * u));
-  const float hits = fmaxf(lone.known, leaves * spheres * __builtin_amdgcn_rcpf(box));
-  return leaves * (2.2f + 0.094f * fminf(hits, (float)GROUP_CAND)) <=
-         lone.base + lone.per_hit * hits;
+  // most groups pay even if every leaf of their blocks is a candidate
+  int blocks = 0;
+  for (int j = 0; j < nodes; ++j)
+    blocks += __popcll(L.blocks[j]);
+  if (limit.pays(64.f * (float)__builtin_amdgcn_readfirstlane(blocks)))
+    return true;
+  const int lane = threadIdx.x & 63;
+  const float4 *boxes = tv.blk + 2 * (size_t)tv.blk_at[0];
+  float part = 0.f;
+  for (int j = 0; j < nodes; ++j)
+    if ((L.blocks[j] >> lane) & 1u)
+    {
+      const size_t id = (size_t)L.node[buffer][j] * 64u + (size_t)lane;
+      part += group_part(g, boxes[2 * id], boxes[2 * id + 1]);
+    }
+  return limit.pays(64.f * wave_uniform(wave_sum(part)));
 }
 
 // The lane's predicate as the two matrix operands (columns 0-31 and 32-63
@@ -418,12 +458,13 @@ AXB_D void group_leaves(const TreeView &tv, const GroupLds &L, int nodes, int bu
 }
 
 // All hits of the wavefront's predicates, each lane's in leaf order.  Every
-// lane of the wavefront calls it (inactive ones too).  False: not searched,
-// the lanes have to walk the tree themselves.  SKIP: the value `skip` is not
+// lane of the wavefront calls it (inactive ones too).  False: not searched
+// (limit: WalkCost, LeafLimit or NoLimit), the lanes have to walk the tree
+// themselves.  SKIP: the value `skip` is not
 // reported.
-template <bool SKIP, class Sink>
+template <bool SKIP, class Limit, class Sink>
 AXB_D bool group_walk(const TreeView &tv, GroupLds &L, float x, float y, float z, float r,
-                      float thr, bool active, int32_t skip, const LoneCost &lone, Sink &sink,
+                      float thr, bool active, int32_t skip, Limit limit, Sink &sink,
                       uint32_t &v_int, uint32_t &v_leaf)
 {
   // an infinite radius reaches everything, from an infinite (inactive) centre
@@ -436,13 +477,12 @@ AXB_D bool group_walk(const TreeView &tv, GroupLds &L, float x, float y, float z
   if (!group_reach(x, y, z, r, thr, active, g))
     return false;
   int buffer = 0;
-  float part = 0.f;
   const int nodes =
-      group_blocks(tv, g, L, buffer, v_int, [&](uint64_t m, const float4 &a, const float4 &b) {
-        if ((m >> (threadIdx.x & 63)) & 1u)
-          part += group_part(g, a, b);
-      });
-  if (nodes < 0 || !group_pays(g, 64.f * wave_uniform(wave_sum(part)), r, active, lone))
+      group_blocks(tv, g, L, buffer, v_int, [](uint64_t, const float4 &, const float4 &) {});
+  if (nodes < 0)
+    return false;
+  limit.meet(g, r, active);
+  if (!group_pays(tv, g, L, nodes, buffer, limit))
     return false;
   half4_t col[2];
   group_columns(g, x, y, z, r, active, col);

@@ -97,14 +97,16 @@ struct WsLease
   ~WsLease() { release(); }
 };
 
-// Limits that are normally derived from the device, lowered by tests
-// (axb_debug_set_limits) to run the multi-launch and fallback paths on
-// small inputs.  0 = default.
+// Limits that are normally derived from the device or the tree, set by tests
+// (axb_debug_set_limits, axb_debug_set_search) to run the paths of other
+// inputs on small ones.  0 = default.
 struct Limits
 {
   int64_t knn_batch_max;      // kNN queries per collect launch
   int64_t scratch_rows_bytes; // scratch rows of a buffered CRS query
   int32_t knn_rounds;         // collect rounds before the exact fallback
+  int64_t knn_small;          // kNN queries of a small launch
+  int32_t fill;               // 1 + FILL_*
 };
 Limits debug_limits();
 // hipStreamSynchronize, timed as "host:stream_sync" while profiling.

@@ -82,20 +82,26 @@ __global__ __launch_bounds__(256) void k_spatial(
   }
 }
 
-// What 64 lanes' rope walks cost (LoneCost), fitted to k_spatial at 4 to 1000
-// hits.  Where the leaves lie on surfaces or curves the walks are cheaper for
-// their hits.  A row that is written again is as long as its offsets say.
-// Measured alone / together with no limit / with this one: 10M points in
-// clusters too tight for the query order (sigma 0.0005) 9.5 / 11.6 / 9.1 ms,
-// 16k unsorted predicates, 30 hits 0.32 / 0.57 / 0.24, 1M points on a line,
-// 32 hits 0.71 / 1.45 / 0.69; uniform 10M unchanged (6.8 / 3.6 / 3.6).
+// What 64 lanes' rope walks cost (WalkCost), fitted to k_spatial at 4 to 1000
+// hits: a * (2600 + 400 * hits).  a = 1 for walks over leaves on surfaces and
+// curves, the cheapest for their hits (1M points on a line, 32 hits: alone
+// 0.71, together 1.45 ms; a = 1.5 0.87), and for predicates in no order (16k
+// uniform points, 30 hits: alone 0.32, together 0.57, with the limit 0.24 ms).
+// a = 3 in uneven sets, where wavefronts wait for their longest walk (700k
+// spheres in clusters, first pass: no limit 0.208 ms, a = 3 0.207, 2.5 0.220,
+// 1.1 0.257; 10M points in clusters of sigma 0.0005: alone 9.5, together 11.6,
+// a = 3 8.6, 4 10.0).  In even sets groups always pay, and the limit itself
+// costs (2M lattice points' neighbour lists 0.59 ms, 0.62 with a = 2.2).  A
+// row that is written again is as long as its offsets say.
 template <int MODE>
-AXB_D LoneCost rope_walk_cost(const TreeView &tv, const int64_t *__restrict__ offsets, int64_t q,
-                              bool real)
+AXB_D WalkCost rope_walk_cost(const TreeView &tv, const int64_t *__restrict__ offsets, int64_t q,
+                              bool real, bool ordered)
 {
-  const float a = tv.fill == FILL_THIN ? 1.f : 1.6f;
-  LoneCost c{a * 2600.f, a * 400.f, 0.f};
-  if (MODE == MODE_FILL)
+  const float a = tv.fill == FILL_THIN || !ordered ? 1.f
+                  : tv.fill == FILL_UNEVEN         ? 3.f
+                                                   : 0.f;
+  WalkCost c{a > 0.f ? a * 2600.f : FLT_MAX, a * 400.f, 0.f, 0.f};
+  if (MODE == MODE_FILL && a > 0.f)
     c.known = wave_uniform(wave_max(real ? (float)(offsets[q + 1] - offsets[q]) : 0.f));
   return c;
 }
@@ -134,7 +140,8 @@ __global__ __launch_bounds__(256, 6) void k_spatial_group(
     rw.init(out, offsets, q, buffer);
   uint32_t v_int = 0, v_leaf = 0;
   if (!group_walk<false>(tv, s_group[threadIdx.x >> 6], x, y, z, r, thr, active, -1,
-                         rope_walk_cost<MODE>(tv, offsets, q, real), rw, v_int, v_leaf) &&
+                         rope_walk_cost<MODE>(tv, offsets, q, real, order != nullptr), rw, v_int,
+                         v_leaf) &&
       real)
   {
     const SpatialPred pr = sphere_pred(x, y, z, r);
@@ -593,7 +600,8 @@ __global__ __launch_bounds__(256, 6) void k_nlist_group(TreeView tv, float radiu
       real && fabsf(x) < INFINITY && fabsf(y) < INFINITY && fabsf(z) < INFINITY;
   uint32_t v_int = 0, v_leaf = 0;
   if (!group_walk<true>(tv, s_group[threadIdx.x >> 6], x, y, z, radius, thr, active, (int32_t)q,
-                        rope_walk_cost<MODE>(tv, offsets, q, real), rw, v_int, v_leaf) &&
+                        rope_walk_cost<MODE>(tv, offsets, q, real, order != nullptr), rw, v_int,
+                        v_leaf) &&
       real)
   {
     constexpr uint32_t SL = leaf_slots<GEOM_POINTS>(), SI = internal_slots<F>();
@@ -1442,19 +1450,21 @@ AXB_D float group_row_bound(const uint2 *__restrict__ cand, uint32_t row_at, int
 // lane whose row holds between m and cap of them selects its m nearest; the
 // others search again together: a short row with a larger radius, from its
 // count, a full one within its m-th distance.
-// Lanes left after GROUP_ROUNDS, or after the first round when they are many
-// (a density that differs a lot within the group), search alone as in
-// k_knn_collect.  10M uniform points, k = 16: 9.14 (k_knn_collect) -> 4.29 ms,
-// 13300 vector instructions per wavefront, 79% of the issue rate: about half
-// the exact tests of the ~38 leaves a lane finds, a fifth the selection; five
-// wavefronts per SIMD (six: 4.36 ms, 26 registers spilled).
+// Lanes left after GROUP_ROUNDS, or where another round would be more work
+// (limit), search alone as in k_knn_collect.  EVEN: the radius is guessed
+// from the group's density (spacing: of the leaves), else from each lane's
+// own (spacing: leaves per query).  10M uniform points, k = 16: 9.14
+// (k_knn_collect) -> 4.25 ms, 13300 vector instructions per wavefront, 79%
+// of the issue rate: about half the exact tests of the ~38 leaves a lane
+// finds, a fifth the selection; five wavefronts per SIMD (six: 4.36 ms, 26
+// registers spilled).  The limit costs 0.14 ms there, so batches over uniform
+// leaves, where every group pays, go without.
 constexpr int GROUP_ROUNDS = 6;
-template <int F, int K, bool TOGETHER>
+template <int F, int K, bool EVEN, class Limit>
 __global__ __launch_bounds__(256, K <= 16 ? 5 : (K <= 32 ? 4 : 2)) void k_knn_collect_group(
     TreeView tv, const float *__restrict__ pts, int64_t t0, int64_t tn, int k, float want,
-    float spacing, int W, float shrink, const uint32_t *__restrict__ order,
-    uint2 *__restrict__ cand, int cap,
-    int max_rounds, uint32_t *__restrict__ ovf, uint32_t *__restrict__ ovf_n,
+    float spacing, Limit limit, int W, float shrink, const uint32_t *__restrict__ order,
+    uint2 *__restrict__ cand, int cap, int max_rounds, uint32_t *__restrict__ ovf, uint32_t *__restrict__ ovf_n,
     int32_t *__restrict__ oi, float *__restrict__ od)
 {
   __shared__ GroupLds s_group[4];
@@ -1478,9 +1488,8 @@ __global__ __launch_bounds__(256, K <= 16 ? 5 : (K <= 32 ? 4 : 2)) void k_knn_co
   const int lane = threadIdx.x & 63;
   bool guessed = max_rounds > 0 && __ballot(pending) != 0;
   if (guessed)
-    guessed = TOGETHER ? group_guess_radius(tv, L, x, y, z, pending, want, spacing, r, v_int,
-                                            v_leaf)
-                       : group_guess_own_radius(tv, L, x, y, z, pending, want, spacing, r, v_int);
+    guessed = EVEN ? group_guess_radius(tv, L, x, y, z, pending, want, spacing, r, v_int, v_leaf)
+                   : group_guess_own_radius(tv, L, x, y, z, pending, want, spacing, r, v_int);
   if (guessed)
   {
 #pragma unroll 1
@@ -1488,8 +1497,8 @@ __global__ __launch_bounds__(256, K <= 16 ? 5 : (K <= 32 ? 4 : 2)) void k_knn_co
     {
       ++rounds;
       row.cnt = 0;
-      if (!group_walk<false>(tv, L, x, y, z, r, sqrt_threshold(r), pending, -1,
-                             LoneCost{FLT_MAX, 0.f, 0.f}, row, v_int, v_leaf))
+      if (!group_walk<false>(tv, L, x, y, z, r, sqrt_threshold(r), pending, -1, limit, row,
+                             v_int, v_leaf))
         break;
       wave_lds_order();
       if (pending)
@@ -1503,8 +1512,7 @@ __global__ __launch_bounds__(256, K <= 16 ? 5 : (K <= 32 ? 4 : 2)) void k_knn_co
         else if (row.cnt < m)
           r *= fminf(fmaxf(approx_cbrt(want / (float)(row.cnt > 0 ? row.cnt : 1)), 1.26f), 2.5f);
       }
-      const uint64_t open = __ballot(pending);
-      if (open == 0 || (!TOGETHER && __popcll(open) > 12))
+      if (__ballot(pending) == 0)
         break;
       if (__ballot(pending && row.cnt > cap))
       {
@@ -1993,22 +2001,42 @@ int knn_row_capacity(int k, int n) { return knn_shape(k, n).cap; }
 // Leaves the group search aims at for k nearest: a count that is Poisson
 // around k + 4 sqrt(k) + 4 falls below k once in ~10^4.
 static float knn_group_want(int k) { return (float)k + 4.f * std::sqrt((float)k) + 4.f; }
-// Up to this many queries a launch is as long as its slowest wavefronts: a
-// group then goes on together until its last lane is done, from the group's
-// density.  With more, lanes take their own density, and when more than a
-// few of them need another round they walk alone, which costs less work
-// (clustered points, k = 10: 100k queries 0.29 ms together, 0.57 alone; 4M
-// queries 4.6 ms together, 3.3 alone; uniform 0.10 / 0.13 and 1.6 / 1.7).
-constexpr int64_t KNN_TOGETHER_MAX = 300000;
+// Up to this many queries a launch is as long as its slowest wavefronts.
+static int64_t knn_small()
+{
+  const int64_t lim = debug_limits().knn_small;
+  return lim > 0 ? lim : 300000;
+}
+// The most candidates a group may search: what they cost (group_cost) is then
+// that of 64 lanes' own walks, about 8800 + 1360 vector instructions per leaf
+// wanted.
+static LeafLimit knn_leaf_limit(int k)
+{
+  const float want = knn_group_want(k);
+  return LeafLimit{(8800.f + 1360.f * want) /
+                   (2.2f + 0.094f * std::min(want, (float)GROUP_CAND))};
+}
 // Queries of a point tree that are sorted along the Hilbert curve search in
 // groups when they are not fewer than half the points (a group of sparser
 // ones sees too many leaves: 1M clustered points, 130k queries, k = 10 0.61
 // -> 0.83 ms), for k >= 2 (the nearest one of 4M uniform points: 0.90 ms
-// alone, 1.03 in groups).
+// alone, 1.03 in groups), and where the leaves fill space evenly enough for
+// the guessed radius to be right (TreeView::fill).  Calls, alone / in groups
+// of k_knn_collect_group<.., NoLimit>, in ms:
+//   even         1M uniform, k = 10           1.02 / 0.65
+//                250k normal, k = 10          0.72 / 0.71
+//   uneven       1M on a sphere, k = 10       1.06 / 1.23, k = 24 2.12 / 1.62
+//                1M in 1000 clusters, k = 10  1.49 / 1.52, k = 24 3.21 / 2.42
+//                50k on a sphere, k = 5       0.35 / 0.35, k = 10 0.44 / 0.44
+//                  (with the limit                   0.29              0.31)
+//   thin         1M on a line, k = 24         2.04 / 4.99
+//                50k in 20 clusters, k = 10   0.68 / 1.94, k = 24 1.55 / 2.70
 bool knn_group_rule(const TreeView &tv, int64_t nq, int k)
 {
   return tv.leaves && k >= 2 && k <= 64 && nq * 2 >= tv.n &&
-         (float)tv.n >= 8.f * knn_group_want(k);
+         (float)tv.n >= 8.f * knn_group_want(k) &&
+         (tv.fill >= FILL_EVEN ||
+          (tv.fill == FILL_UNEVEN && (k >= 20 || (k >= 8 && nq <= knn_small()))));
 }
 
 template <int F, int G, int K>
@@ -2029,7 +2057,10 @@ static hipError_t knn_run(const TreeView &tv, const float *pts, int64_t nq, int 
     vol *= std::max(tv.scene.hi[d] - tv.scene.lo[d], 1e-3f * longest);
   const float spacing = std::cbrt(vol / (float)tv.n);
   const float per_query = (float)tv.n / (float)nq;
-  const bool together = nq <= KNN_TOGETHER_MAX;
+  // small launches over uniform leaves guess from the group's density: fewer
+  // groups need a second round (calls of 250k points, k = 10: 0.28 ms, 0.34
+  // from the lanes' own; normal ones, k = 5, 0.55 / 0.48)
+  const bool small = nq <= knn_small();
   for (int64_t t0 = 0; e == hipSuccess && t0 < nq; t0 += ws.batch)
   {
     const int64_t tn = std::min(ws.batch, nq - t0);
@@ -2037,14 +2068,18 @@ static hipError_t knn_run(const TreeView &tv, const float *pts, int64_t nq, int 
     if constexpr (G == GEOM_POINTS)
     {
       group = order && knn_group_rule(tv, nq, k);
-      if (group && together)
-        AXB_LAUNCH((k_knn_collect_group<F, K, true>), dim3(grid_of(tn)), dim3(256), 0, s, tv, pts, t0,
-                   tn, k, want, spacing, sh.W, sh.shrink, order, ws.cand, sh.cap, rounds, ws.ovf,
-                   ws.ovf_n, oi, od);
+      if (group && tv.fill == FILL_UNIFORM && small)
+        AXB_LAUNCH((k_knn_collect_group<F, K, true, NoLimit>), dim3(grid_of(tn)), dim3(256), 0, s,
+                   tv, pts, t0, tn, k, want, spacing, NoLimit{}, sh.W, sh.shrink, order, ws.cand,
+                   sh.cap, rounds, ws.ovf, ws.ovf_n, oi, od);
+      else if (group && tv.fill == FILL_UNIFORM)
+        AXB_LAUNCH((k_knn_collect_group<F, K, false, NoLimit>), dim3(grid_of(tn)), dim3(256), 0, s,
+                   tv, pts, t0, tn, k, want, per_query, NoLimit{}, sh.W, sh.shrink, order, ws.cand,
+                   sh.cap, rounds, ws.ovf, ws.ovf_n, oi, od);
       else if (group)
-        AXB_LAUNCH((k_knn_collect_group<F, K, false>), dim3(grid_of(tn)), dim3(256), 0, s, tv, pts, t0,
-                   tn, k, want, per_query, sh.W, sh.shrink, order, ws.cand, sh.cap, rounds,
-                   ws.ovf, ws.ovf_n, oi, od);
+        AXB_LAUNCH((k_knn_collect_group<F, K, false, LeafLimit>), dim3(grid_of(tn)), dim3(256), 0,
+                   s, tv, pts, t0, tn, k, want, per_query, knn_leaf_limit(k), sh.W, sh.shrink,
+                   order, ws.cand, sh.cap, rounds, ws.ovf, ws.ovf_n, oi, od);
     }
     if (group)
       ;

@@ -220,3 +220,68 @@ def test_cost_of_a_group_at_any_scale(scale):
     p = (synthetic.uniform_points(20000, 3) * np.float32(scale)).astype(np.float32)
     r = np.float32(synthetic.radius_for_neighbours(20000, 30) * scale)
     assert _leaves_per_query(p, _spheres(p, r), True) < 40
+
+
+def _knn_kernels(points, k, nq=None):
+    tree = ax.BVH(torch.from_numpy(points).cuda(), node_format="q16")
+    q = ax.make_nearest(torch.from_numpy(points[:nq]), k)
+    with ax.profile(timing=True) as prof:
+        tree.query(q)
+    return [n for n in prof.kernels if "k_knn_collect" in n]
+
+
+@pytest.mark.parametrize("k,grouped", [(2, "uniform"), (5, "uniform"), (8, "uniform sphere"),
+                                       (24, "uniform sphere")])
+def test_nearest_in_groups_where_leaves_fill_space(k, grouped):
+    n = 40000
+    g = np.random.default_rng(5)
+    u = g.normal(size=(n, 3))
+    t = g.uniform(0, 40, n)
+    line = np.full((n, 3), 0.5)
+    line[:, 0] = g.uniform(size=n)
+    centres = g.uniform(size=(20, 3))
+    sets = dict(uniform=g.uniform(size=(n, 3)), sphere=u / np.linalg.norm(u, axis=1)[:, None],
+                helix=np.stack([np.cos(t), np.sin(t), t / 40], 1), line=line,
+                clusters=centres[np.arange(n) % 20] + 0.001 * u)
+    for name, p in sets.items():
+        p = p.astype(np.float32)
+        kernels = _knn_kernels(p, k)
+        assert len(kernels) == 1
+        assert ("k_knn_collect_group" in kernels[0]) == (name in grouped.split()), name
+        _check_nearest(p, p[:2000].copy(), k)
+        _check_nearest(p, p, k)
+
+
+@pytest.mark.parametrize("fill", [0, 1, 2, 3])
+@pytest.mark.parametrize("k", [2, 3, 5, 8, 13, 16, 17, 24, 32, 33, 64])
+def test_nearest_over_every_route(k, fill):
+    # uneven density, duplicates, ties and queries without an answer, through
+    # each guess of the radius and as small and as large launches
+    g = np.random.default_rng(k)
+    p = g.uniform(size=(7000, 3))
+    p[:3000] = g.uniform(size=(30, 3))[np.arange(3000) % 30]
+    p[:3000] += 10.0 ** g.uniform(-4, -1, (3000, 1)) * g.normal(size=(3000, 3))
+    p[3000:3500, 1:] = 0.5
+    p[3500:3600] = p[3500]
+    a = np.arange(12) / 12.0
+    p[4000:4000 + 1728] = np.stack(np.meshgrid(a, a, a, indexing="ij"), -1).reshape(-1, 3)
+    p = p.astype(np.float32)
+    q = np.concatenate([p, synthetic.uniform_points(999, k) * np.float32(2) - np.float32(0.5)])
+    t = oracle.Tree(p, 0)
+    o_ref, i_ref, d_ref = t.query_knn(q, k)
+    bad = q.copy()
+    bad[::37, 1] = np.nan
+    bad[5::41, 2] = np.inf
+    ref_bad = ax.BruteForce(torch.from_numpy(p).cuda()).query(
+        ax.make_nearest(torch.from_numpy(bad), k))[0].reshape(-1, k)
+    keep = torch.from_numpy(np.isfinite(bad).all(1)).cuda()
+    tree = ax.BVH(torch.from_numpy(p).cuda(), node_format="fp32" if k % 2 else "q16")
+    for small in (1, 1 << 30):
+        for limits in (dict(), dict(knn_batch_max=777)):
+            with ax.debug_search(knn_small=small, fill=fill), ax.debug_limits(**limits):
+                i, o, d = tree.query(ax.make_nearest(torch.from_numpy(q), k),
+                                     return_distances=True)
+                b = tree.query(ax.make_nearest(torch.from_numpy(bad), k))[0].reshape(-1, k)
+            np.testing.assert_array_equal(i.cpu().numpy(), i_ref)
+            np.testing.assert_array_equal(d.cpu().numpy().view(np.uint32), d_ref.view(np.uint32))
+            assert torch.equal(b[keep], ref_bad[keep])
