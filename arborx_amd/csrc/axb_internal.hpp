@@ -146,15 +146,17 @@ hipError_t radix_sort_pairs_u32(uint32_t *keys0, uint32_t *keys1,
                                 int passes, uint32_t *hist, void *workspace,
                                 uint32_t *err, hipStream_t stream);
 // The same for the build's 63-bit Morton codes; hist holds the digits' counts
-// from bit sort_hist_shift(n) on, words SORT_RUN_WORDS scratch words.  Large batches
-// sort by the top 32 bits first (four passes of 24 bytes per key instead of
-// eight), put the runs of equal top halves right one by one, and run the
-// eight passes only when a run is too long (kernels behind a device flag, no
-// copy to the host; their empty launches cost ~25 us, about what is saved at
-// 0.3-0.5M keys: calls 0.74 / 0.72 ms at 350k, 0.85 / 0.82 at 1M, 1.14 / 0.98
-// at 2.2M and 2.60 / 2.18 at 10M uniform points, 1.66 / 1.55 at 5M clustered
-// ones).
-constexpr int SORT_RUN_WORDS = 3;
+// from bit sort_hist_shift(n) on, words SORT_RUN_WORDS scratch words.  Large
+// batches sort by the top 32 bits first (four passes of 24 bytes per key
+// instead of eight) and put the runs of equal top halves right one by one;
+// the eight passes run instead when a sample shows that keys crowd into cells,
+// and after the four when a run is too long (kernels behind device flags, no
+// copy to the host).  Builds with eight passes / with this: uniform points
+// 0.48 / 0.42 ms at 524k, 0.54 / 0.47 at 1M, 0.78 / 0.64 at 2.2M, 2.20 / 1.77
+// at 10M; 1000 clusters of sigma 0.0001, where the eight passes run, 0.61 /
+// 0.65 at 1M and 2.41 / 2.45 at 10M.  (350k uniform points would gain too, 0.44
+// / 0.39.)
+constexpr int SORT_RUN_WORDS = 6;
 constexpr int64_t SORT_TOP_FIRST_MIN = int64_t(1) << 19;
 inline bool sort_top_first(int64_t n) { return n >= SORT_TOP_FIRST_MIN; }
 inline int sort_hist_shift(int64_t n) { return sort_top_first(n) ? 31 : 0; }

@@ -130,10 +130,13 @@ __global__ __launch_bounds__(SORT_BLOCK) void k_onesweep(
     const uint32_t *__restrict__ digit_offset,
     const uint32_t *__restrict__ trivial, uint32_t *__restrict__ status,
     uint32_t *__restrict__ tile_counter, uint32_t *__restrict__ err,
-    const uint32_t *__restrict__ gate)
+    const uint32_t *__restrict__ gate, const uint32_t *__restrict__ no_vals)
 {
   if (gate && *gate == 0u)
     return;
+  // (no_vals: given and not zero, the values are the positions)
+  if (no_vals && *no_vals != 0u)
+    vin = nullptr;
   constexpr int WAVES = SORT_BLOCK / 64;
   __shared__ uint32_t s_tile;
   __shared__ uint32_t s_whist[WAVES][256];
@@ -451,13 +454,14 @@ inline int fill_grid(int64_t n)
 }
 
 // Stable LSD sort by the digits of bits [shift0, shift0 + 8 passes).  vals0
-// holds the values when have_vals, else they are the positions.  gate: as in
-// the kernels (a gated sort makes its own histograms).
+// holds the values when have_vals (and not *no_vals), else they are the
+// positions.  gate: as in the kernels.
 template <class K>
 hipError_t radix_sort_pairs(K *keys0, K *keys1, uint32_t *vals0,
                             uint32_t *vals1, int64_t n, int passes, int shift0, bool have_vals,
                             uint32_t *hist, void *workspace, uint32_t *err,
-                            hipStream_t stream, const uint32_t *gate)
+                            hipStream_t stream, const uint32_t *gate,
+                            const uint32_t *no_vals = nullptr)
 {
   const int64_t tiles = div_up(n, SORT_TILE);
   // workspace layout: [hist passes*256][trivial passes][counters passes]
@@ -488,7 +492,8 @@ hipError_t radix_sort_pairs(K *keys0, K *keys1, uint32_t *vals0,
     AXB_LAUNCH(k_onesweep<K>, dim3((unsigned)tiles), dim3(SORT_BLOCK),
                        0, stream, kin, vin, kout, vout, n, shift0 + 8 * p,
                        hist + p * 256, trivial + p,
-                       status + (size_t)p * tiles * 256, counters + p, err, gate);
+                       status + (size_t)p * tiles * 256, counters + p, err, gate,
+                       p == 0 ? no_vals : (const uint32_t *)nullptr);
     K *kt = kin;
     kin = kout;
     kout = kt;
@@ -502,18 +507,97 @@ hipError_t radix_sort_pairs(K *keys0, K *keys1, uint32_t *vals0,
 // Keys sorted by their top 32 bits (shift HI_SHIFT) are sorted altogether
 // but for runs of equal top halves whose low halves are out of order.  An
 // inversion (a neighbour with the same top half and a smaller key) that is
-// the first of its run lists the run: up to RUN_SHORT keys for a thread, up
-// to RUN_LONG for a block.  A longer one, or one whose first inversion comes
-// after RUN_SHORT keys in order, opens the gate of the full sort.  Runs of
-// equal keys hold no inversions.  k_find_runs takes 0.031 ms for the keys of
-// 10M uniform points, each of the four passes saved 0.12 to 0.15 ms.
+// the first of its run lists the run: up to RUN_TINY keys for a thread, up to
+// RUN_SHORT for a wavefront, up to RUN_LONG for a block.  A longer one, or one
+// whose first inversion comes after RUN_SHORT keys in order, opens the gate of
+// the full sort.  Runs of equal keys hold no inversions.  k_find_runs takes
+// 0.031 ms for the keys of 10M uniform points, each of the four passes saved
+// 0.12 to 0.15 ms.
 constexpr int HI_SHIFT = 31;
+constexpr int RUN_TINY = 8;
 constexpr int RUN_SHORT = 64;
 constexpr int RUN_LONG = 4096;
 struct RunWords
 {
-  uint32_t shorts, gate, longs;
+  uint32_t tinies, shorts, longs; // runs on the lists
+  uint32_t gate;                  // the full sort runs
+  uint32_t top;                   // the sort by the top halves runs
+  uint32_t crowded;               // it does not (no permutation yet)
 };
+static_assert(sizeof(RunWords) == SORT_RUN_WORDS * 4, "scratch words");
+
+// A look at SAMPLE keys before the sort, for whether the full sort runs at
+// once, without the four passes by the top halves.  A sampled key matches when
+// an earlier one has its top half but not its low half; where keys crowd into
+// cells there are about SAMPLE^2 / 2 times the sum of the squared parts of the
+// keys in a cell of them.  From SAMPLE_MATCHES on, putting the runs right
+// costs more than the passes saved (1000 clusters of sigma 0.001, 30 to 40
+// matches: 10M points 2.35 ms with eight passes, 2.66 with four, 1M 0.58 /
+// 0.59; of sigma 0.0001 1M 0.61 / 0.73; of sigma 0.01, no match, 2.23 / 1.80
+// and 0.56 / 0.49), and `crowd` matches in one cell stand for a run of 1.5
+// RUN_LONG (SAMPLE L / n of a run of L), too long for a block.  Also clears
+// the words.
+constexpr uint32_t SAMPLE_MATCHES = 24;
+constexpr int SAMPLE = 4096, SAMPLE_SLOTS = 8192, SAMPLE_COUNTS = 2048;
+inline uint32_t sample_crowd(int64_t n)
+{
+  const int64_t c = (int64_t)SAMPLE * (RUN_LONG + RUN_LONG / 2) / n;
+  return (uint32_t)(c < 3 ? 3 : c);
+}
+__global__ __launch_bounds__(1024) void k_sample_runs(const uint64_t *__restrict__ keys,
+                                                      int64_t n, uint32_t crowd, RunWords *w)
+{
+  constexpr uint32_t EMPTY = ~0u;
+  constexpr int PER = SAMPLE / 1024;
+  __shared__ __align__(16) uint32_t s_top[SAMPLE_SLOTS], s_count[SAMPLE_COUNTS];
+  __shared__ uint32_t s_low[SAMPLE_SLOTS];
+  __shared__ uint32_t s_crowded, s_matches;
+  uint64_t k[PER];
+#pragma unroll
+  for (int j = 0; j < PER; ++j)
+  {
+    // one key of each part of the input, at a different place in each
+    const uint32_t s = (uint32_t)j * 1024u + threadIdx.x;
+    const uint64_t at = (uint64_t)s * 65536u + ((s * 40503u) & 65535u);
+    k[j] = keys[at * (uint64_t)n / ((uint64_t)SAMPLE * 65536u)];
+  }
+  for (int j = threadIdx.x; j < SAMPLE_SLOTS / 4; j += 1024)
+    ((uint4 *)s_top)[j] = make_uint4(EMPTY, EMPTY, EMPTY, EMPTY);
+  for (int j = threadIdx.x; j < SAMPLE_COUNTS / 4; j += 1024)
+    ((uint4 *)s_count)[j] = make_uint4(0u, 0u, 0u, 0u);
+  if (threadIdx.x == 0)
+    s_crowded = 0u, s_matches = 0u;
+  __syncthreads();
+  uint32_t slot[PER];
+#pragma unroll
+  for (int j = 0; j < PER; ++j)
+  {
+    uint32_t top = (uint32_t)(k[j] >> HI_SHIFT);
+    top = top == EMPTY ? EMPTY - 1u : top;
+    uint32_t h = (top * 2654435761u) >> 19; // half of the slots stay empty
+    while (true)
+    {
+      const uint32_t was = atomicCAS(&s_top[h], EMPTY, top);
+      if (was == EMPTY)
+        s_low[h] = (uint32_t)k[j]; // the first of its top half
+      if (was == EMPTY || was == top)
+        break;
+      h = (h + 1u) & (SAMPLE_SLOTS - 1u);
+    }
+    slot[j] = h;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int j = 0; j < PER; ++j)
+    if (((s_low[slot[j]] ^ (uint32_t)k[j]) & ((1u << HI_SHIFT) - 1u)) != 0u &&
+        (atomicAdd(&s_count[slot[j] & (SAMPLE_COUNTS - 1)], 1u) + 1u >= crowd ||
+         atomicAdd(&s_matches, 1u) + 1u >= SAMPLE_MATCHES))
+      s_crowded = 1u;
+  __syncthreads();
+  if (threadIdx.x == 0)
+    *w = RunWords{0u, 0u, 0u, s_crowded, s_crowded ^ 1u, s_crowded};
+}
+
 // The first inversion of a run at i: its run [b, e); e - b > RUN_LONG stands
 // for the gate.  False: no inversion at i, or not its run's first.
 AXB_D bool run_at(const uint64_t *__restrict__ keys, int64_t n, int64_t i, int64_t &b, int64_t &e)
@@ -552,7 +636,7 @@ AXB_D bool run_at(const uint64_t *__restrict__ keys, int64_t n, int64_t i, int64
   }
   return true;
 }
-// shorts: starts of the short runs; longs: {start, end} of the long ones.  A
+// tinies: starts of the tiny runs; shorts, longs: {start, end} of the others.  A
 // block gathers the runs of RUN_TILE keys in LDS and takes its place in the
 // lists with one atomic each.  All of them meet in one word, 20 to 27 ns an
 // atomic, and bound the kernel where most tiles hold a run: one per run took
@@ -564,14 +648,17 @@ constexpr int RUN_BLOCK = 1024;
 constexpr int RUN_AHEAD = 8;
 static_assert(RUN_TILE % (RUN_BLOCK * RUN_AHEAD) == 0, "whole steps");
 __global__ __launch_bounds__(RUN_BLOCK) void k_find_runs(const uint64_t *__restrict__ keys, int64_t n,
-                                                   uint32_t *__restrict__ shorts,
+                                                   uint32_t *__restrict__ tinies,
+                                                   uint2 *__restrict__ shorts,
                                                    uint2 *__restrict__ longs, RunWords *w)
 {
-  // a run on the list has an inversion, two keys, in the tile
-  __shared__ uint32_t s_short[RUN_TILE / 2 + 1];
+  // a run on the list has an inversion, two keys, in the tile, and all but the
+  // last of the tile end in it
+  __shared__ uint32_t s_tiny[RUN_TILE / 2 + 1];
+  __shared__ uint2 s_short[RUN_TILE / RUN_TINY + 2];
   __shared__ uint2 s_long[RUN_TILE / RUN_SHORT + 2];
-  __shared__ uint32_t s_n[4];
-  if (threadIdx.x < 4)
+  __shared__ uint32_t s_n[6];
+  if (threadIdx.x < 6)
     s_n[threadIdx.x] = 0u;
   __syncthreads();
   const int64_t base = (int64_t)blockIdx.x * RUN_TILE;
@@ -597,10 +684,12 @@ __global__ __launch_bounds__(RUN_BLOCK) void k_find_runs(const uint64_t *__restr
         int64_t b, e;
         if (!run_at(keys, n, base + j + RUN_BLOCK * (__ffs(inversions) - 1), b, e))
           continue;
-        if (e - b <= RUN_SHORT)
-          s_short[atomicAdd(&s_n[0], 1u)] = (uint32_t)b;
+        if (e - b <= RUN_TINY)
+          s_tiny[atomicAdd(&s_n[0], 1u)] = (uint32_t)b;
+        else if (e - b <= RUN_SHORT)
+          s_short[atomicAdd(&s_n[1], 1u)] = make_uint2((uint32_t)b, (uint32_t)e);
         else if (e - b <= RUN_LONG)
-          s_long[atomicAdd(&s_n[1], 1u)] = make_uint2((uint32_t)b, (uint32_t)e);
+          s_long[atomicAdd(&s_n[2], 1u)] = make_uint2((uint32_t)b, (uint32_t)e);
         else
           st_agent(&w->gate, 1u);
       }
@@ -608,41 +697,97 @@ __global__ __launch_bounds__(RUN_BLOCK) void k_find_runs(const uint64_t *__restr
   __syncthreads();
   if (threadIdx.x == 0)
   {
-    s_n[2] = s_n[0] ? atomicAdd(&w->shorts, s_n[0]) : 0u;
-    s_n[3] = s_n[1] ? atomicAdd(&w->longs, s_n[1]) : 0u;
+    s_n[3] = s_n[0] ? atomicAdd(&w->tinies, s_n[0]) : 0u;
+    s_n[4] = s_n[1] ? atomicAdd(&w->shorts, s_n[1]) : 0u;
+    s_n[5] = s_n[2] ? atomicAdd(&w->longs, s_n[2]) : 0u;
   }
   __syncthreads();
   for (uint32_t j = threadIdx.x; j < s_n[0]; j += RUN_BLOCK)
-    shorts[s_n[2] + j] = s_short[j];
+    tinies[s_n[3] + j] = s_tiny[j];
   for (uint32_t j = threadIdx.x; j < s_n[1]; j += RUN_BLOCK)
-    longs[s_n[3] + j] = s_long[j];
+    shorts[s_n[4] + j] = s_short[j];
+  for (uint32_t j = threadIdx.x; j < s_n[2]; j += RUN_BLOCK)
+    longs[s_n[5] + j] = s_long[j];
 }
 
-// Stable insertion sort of the listed runs, a thread each.
+// Stable insertion sort of a tiny run by a thread.
+AXB_D void fix_tiny_run(uint64_t *keys, uint32_t *vals, int64_t n, int64_t b)
+{
+  const uint64_t top = keys[b] >> HI_SHIFT;
+  for (int64_t j = b + 1; j < n && j - b < RUN_TINY; ++j)
+  {
+    const uint64_t k = keys[j];
+    if ((k >> HI_SHIFT) != top)
+      break;
+    const uint32_t v = vals[j];
+    int64_t h = j;
+    while (h > b && keys[h - 1] > k)
+    {
+      keys[h] = keys[h - 1], vals[h] = vals[h - 1];
+      --h;
+    }
+    keys[h] = k, vals[h] = v;
+  }
+}
+
+// A short run by a wavefront: bitonic sort in registers of (low half,
+// position), which is the stable order.
+AXB_D void fix_short_run(uint64_t *keys, uint32_t *vals, uint2 be)
+{
+  static_assert(RUN_SHORT == 64, "a key per lane");
+  constexpr uint64_t LOW = (1ull << HI_SHIFT) - 1ull;
+  const int lane = threadIdx.x & 63;
+  const bool in = lane < (int)(be.y - be.x); // at most RUN_SHORT
+  unsigned long long k = ~0ull;
+  uint64_t top = 0;
+  uint32_t v = 0;
+  if (in)
+  {
+    const uint64_t key = keys[be.x + lane];
+    v = vals[be.x + lane];
+    top = key & ~LOW;
+    k = ((key & LOW) << 6) | (uint64_t)lane;
+  }
+#pragma unroll
+  for (int span = 2; span <= 64; span *= 2)
+#pragma unroll
+    for (int stride = span / 2; stride > 0; stride /= 2)
+    {
+      const unsigned long long o = __shfl_xor(k, stride, 64);
+      const bool smaller = ((lane & stride) == 0) == ((lane & span) == 0);
+      k = (o < k) == smaller ? o : k;
+    }
+  const uint32_t from = (uint32_t)__shfl((int)v, (int)(k & 63ull), 64);
+  if (in)
+  {
+    keys[be.x + lane] = top | (k >> 6);
+    vals[be.x + lane] = from;
+  }
+}
+
+// The tiny runs by the first TINY_BLOCKS blocks, the short ones by the others.
+// 10M points in 1000 clusters of sigma 0.001, runs of 10 to 60 keys: 2.9 ms
+// with a thread per short run, 0.11 here.
+constexpr int TINY_BLOCKS = 256, SHORT_BLOCKS = 1024;
 __global__ __launch_bounds__(256) void k_fix_runs(uint64_t *keys, uint32_t *vals, int64_t n,
-                                                  const uint32_t *__restrict__ list,
+                                                  const uint32_t *__restrict__ tinies,
+                                                  const uint2 *__restrict__ shorts,
                                                   const RunWords *__restrict__ w)
 {
-  const uint32_t runs = w->shorts;
-  for (uint32_t r = blockIdx.x * blockDim.x + threadIdx.x; r < runs;
-       r += gridDim.x * blockDim.x)
+  if (w->gate)
+    return;
+  if (blockIdx.x < TINY_BLOCKS)
   {
-    const int64_t b = list[r];
-    const uint64_t top = keys[b] >> HI_SHIFT;
-    for (int64_t j = b + 1; j < n && j - b <= RUN_SHORT; ++j)
-    {
-      const uint64_t k = keys[j];
-      if ((k >> HI_SHIFT) != top)
-        break;
-      const uint32_t v = vals[j];
-      int64_t h = j;
-      while (h > b && keys[h - 1] > k)
-      {
-        keys[h] = keys[h - 1], vals[h] = vals[h - 1];
-        --h;
-      }
-      keys[h] = k, vals[h] = v;
-    }
+    const uint32_t runs = w->tinies;
+    for (uint32_t r = blockIdx.x * 256u + threadIdx.x; r < runs; r += TINY_BLOCKS * 256u)
+      fix_tiny_run(keys, vals, n, tinies[r]);
+  }
+  else
+  {
+    const uint32_t runs = w->shorts;
+    for (uint32_t r = (blockIdx.x - TINY_BLOCKS) * 4u + threadIdx.x / 64u; r < runs;
+         r += SHORT_BLOCKS * 4u)
+      fix_short_run(keys, vals, shorts[r]);
   }
 }
 
@@ -710,23 +855,23 @@ hipError_t sort_keys63(uint64_t *keys0, uint64_t *keys1, uint32_t *vals0, uint32
   if (!sort_top_first(n))
     return radix_sort_pairs<uint64_t>(keys0, keys1, vals0, vals1, n, 8, 0, false, hist,
                                       workspace, err, stream, nullptr);
-  hipError_t e = fill_u32(words, 0u, SORT_RUN_WORDS, stream);
-  if (e == hipSuccess)
-    e = radix_sort_pairs<uint64_t>(keys0, keys1, vals0, vals1, n, 4, HI_SHIFT, false, hist,
-                                   workspace, err, stream, nullptr);
+  RunWords *w = (RunWords *)words;
+  AXB_LAUNCH(k_sample_runs, dim3(1), dim3(1024), 0, stream, keys0, n, sample_crowd(n), w);
+  hipError_t e = radix_sort_pairs<uint64_t>(keys0, keys1, vals0, vals1, n, 4, HI_SHIFT, false,
+                                            hist, workspace, err, stream, &w->top);
   if (e != hipSuccess)
     return e;
-  // the other buffers hold the lists (a short run has at least two keys, a
-  // long one 65)
-  RunWords *w = (RunWords *)words;
-  uint2 *longs = (uint2 *)keys1;
-  AXB_LAUNCH(k_find_runs, dim3((unsigned)div_up(n, RUN_TILE)), dim3(RUN_BLOCK), 0, stream, keys0, n, vals1,
-             longs, w);
-  AXB_LAUNCH(k_fix_runs, dim3(256), dim3(256), 0, stream, keys0, vals0, n, vals1, w);
+  // the other buffers hold the lists (a tiny run has at least two keys, a
+  // short one 9, a long one 65)
+  uint2 *shorts = (uint2 *)keys1, *longs = (uint2 *)keys1 + n / 2;
+  AXB_LAUNCH(k_find_runs, dim3((unsigned)div_up(n, RUN_TILE)), dim3(RUN_BLOCK), 0, stream, keys0, n,
+             vals1, shorts, longs, w);
+  AXB_LAUNCH(k_fix_runs, dim3(TINY_BLOCKS + SHORT_BLOCKS), dim3(256), 0, stream, keys0, vals0, n,
+             vals1, shorts, w);
   AXB_LAUNCH(k_fix_long_runs, dim3(512), dim3(256), 0, stream, keys0, vals0, longs, w);
   // nothing to do unless the gate is open
   return radix_sort_pairs<uint64_t>(keys0, keys1, vals0, vals1, n, 8, 0, true, nullptr,
-                                    workspace, err, stream, &w->gate);
+                                    workspace, err, stream, &w->gate, &w->crowded);
 }
 hipError_t radix_sort_pairs_u32(uint32_t *keys0, uint32_t *keys1,
                                 uint32_t *vals0, uint32_t *vals1, int64_t n,

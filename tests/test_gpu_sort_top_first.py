@@ -51,3 +51,29 @@ def test_permutation_is_the_stable_sort(kind):
     e = tree.export_topology()
     np.testing.assert_array_equal(e["perm"].cpu().numpy().view(np.uint32), perm)
     np.testing.assert_array_equal(e["keys"].cpu().numpy().view(np.uint64), codes[perm])
+
+
+@pytest.mark.parametrize("longest", [4096, 4097, 400000])
+def test_runs_at_the_edges_of_their_kernels(longest):
+    # groups of exactly so many points in a cell of the top half of the codes
+    # among many more far from them; 4097 takes the full sort after the one by
+    # the top halves, 400000 instead of it
+    n = 10_000_000
+    g = np.random.default_rng(longest)
+    sizes = [2, 3, 7, 8, 9, 10, 31, 32, 33, 63, 64, 65, 66, 127, 128, 129, 1000, 4095, longest]
+    sizes = sizes + [s for s in sizes if s < 1000] * 40
+    at = g.permutation(100 ** 3)[:len(sizes)]
+    cell = np.stack([at // 10000, at // 100 % 100, at % 100], 1) * 0.005 + 0.0025
+    p = synthetic.uniform_points(n, 4) * np.float32(0.45) + np.float32(0.55)
+    members = np.repeat(cell, sizes, axis=0) + g.uniform(-1, 1, (sum(sizes), 3)) * 2e-5
+    p[g.permutation(n)[:len(members)]] = members
+    p = np.ascontiguousarray(p, np.float32)
+    codes = oracle.morton64_values(p, oracle.scene_box(p))
+    perm = np.argsort(codes, kind="stable")
+    runs = np.unique(codes[perm] >> np.uint64(31), return_counts=True)[1]
+    # (the largest group may lie on a cell's edge)
+    assert set(sizes) <= set(runs.tolist()) or (longest == 400000 and runs.max() > 50000)
+    tree = ax.BVH(torch.from_numpy(p).cuda(), keep_topology=True)
+    e = tree.export_topology()
+    np.testing.assert_array_equal(e["perm"].cpu().numpy().view(np.uint32), perm)
+    np.testing.assert_array_equal(e["keys"].cpu().numpy().view(np.uint64), codes[perm])
