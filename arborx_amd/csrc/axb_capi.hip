@@ -1518,13 +1518,12 @@ axb_status axb_bvh_neighbor_list(const axb_bvh *t, float radius, int32_t full,
     }
   }
   auto first = [&](int mode, int32_t *out, int32_t B) {
-    return launch_nlist(tv, t->node_format, f, radius, n, order, offsets, out, B, rowof, mode, f,
-                        s);
+    return launch_nlist(tv, t->node_format, f, radius, n, order, offsets, out, B, rowof, mode, s);
   };
   // the overflow list holds leaf positions
   auto fill = [&](const uint32_t *list, int64_t n_list, int32_t *out) {
     return launch_nlist(tv, t->node_format, f, radius, n_list, list ? list : order, offsets, out,
-                        0, nullptr, MODE_FILL, f, s);
+                        0, nullptr, MODE_FILL, s);
   };
   // rows of 96, as for queries: the 2M-atom FCC lattice's ~83 neighbours
   // per row take 5.1 ms with rows of 64 (most rows walked twice), 2.4 ms

@@ -477,13 +477,13 @@ hipError_t launch_compact(const int32_t *buf, int64_t nq, int32_t buffer,
                           const int64_t *offsets, int32_t *out, hipStream_t s);
 hipError_t launch_overflow_list(const uint8_t *over_flags, const uint32_t *order, int64_t nq,
                                 bool emit_index, uint32_t *ovf, uint32_t *ovf_n, hipStream_t s);
-// Neighbour list of a point tree: lane t takes leaf position list[t] (t when
-// list is nullptr); rows are the leaves' values.  group: 64 lanes search
-// together (full lists; the positions are sorted along a curve).  rowof (leaf position ->
-// row) is written when non-null.
+// Neighbour list of a point tree of two or more points: lane t takes leaf
+// position list[t] (t when list is nullptr); rows are the leaves' values.
+// full: 64 lanes search together (the positions are sorted along a curve).
+// rowof (leaf position -> row) is written when non-null.
 hipError_t launch_nlist(const TreeView &tv, int node_format, bool full, float radius, int64_t nl,
                         const uint32_t *list, int64_t *offsets, int32_t *out, int32_t buffer,
-                        uint32_t *rowof, int mode, bool group, hipStream_t s);
+                        uint32_t *rowof, int mode, hipStream_t s);
 // Half -> full neighbour list: counts into cnt (zeroed, n + 1 entries), then
 // after the scan into out_offsets, the fill (cursor: n scratch entries).
 hipError_t launch_h2f_count(const int64_t *offsets, const int32_t *indices, int64_t n,

@@ -532,15 +532,15 @@ __global__ __launch_bounds__(256) void k_make_rays(const float *__restrict__ ori
   }
 }
 
-// Neighbour lists over a point tree (NeighborList.hpp:49-188 semantics):
+// Half neighbour lists over a point tree (NeighborList.hpp:49-188 semantics):
 // lane t takes the leaf at position L = list ? list[t] : t and the sphere
-// {its point, radius}; row ~w (its value) receives the values of the other
-// leaves in the sphere -- all of them (FULL) or only those whose leaf comes
-// before L (half list: HalfTraversal.hpp pairs (earlier, later) land in the
-// later leaf's row).  The half walk covers the slots before L's record,
-// which every ancestor of L precedes and passes (distance 0).  rowof[L] is
-// written in the first pass (leaf position -> row) for the overflow list.
-template <int F, bool FULL, int MODE>
+// {its point, radius}; row ~w (its value) receives the values of the leaves
+// in the sphere that come before L (HalfTraversal.hpp: pairs (earlier, later)
+// land in the later leaf's row).  The walk covers the slots before L's
+// record, which every ancestor of L precedes and passes (distance 0).
+// rowof[L] is written in the first pass (leaf position -> row) for the
+// overflow list.
+template <int F, int MODE>
 __global__ __launch_bounds__(256) void k_nlist(TreeView tv, float radius, int64_t nl,
                                                const uint32_t *__restrict__ list,
                                                int64_t *__restrict__ offsets,
@@ -561,8 +561,7 @@ __global__ __launch_bounds__(256) void k_nlist(TreeView tv, float radius, int64_
   RowWriter<MODE> rw;
   rw.init(out, offsets, q, buffer);
   uint32_t v_int = 0, v_leaf = 0;
-  rope_walk<F, GEOM_POINTS, PRED_SPHERES>(tv, pr, 0u, FULL ? tv.total : self, self, rw, v_int,
-                                          v_leaf);
+  rope_walk<F, GEOM_POINTS, PRED_SPHERES>(tv, pr, 0u, self, self, rw, v_int, v_leaf);
   row_epilogue(tv, rw, offsets, q, v_int, v_leaf);
 }
 
@@ -2399,19 +2398,19 @@ hipError_t launch_overflow_list(const uint8_t *over_flags, const uint32_t *order
   return hipGetLastError();
 }
 
-template <int F, bool FULL>
-static hipError_t launch_nlist_f(const TreeView &tv, float radius, int64_t nl,
+template <int F>
+static hipError_t launch_nlist_half(const TreeView &tv, float radius, int64_t nl,
                                  const uint32_t *list, int64_t *offsets, int32_t *out,
                                  int32_t buffer, uint32_t *rowof, int mode, hipStream_t s)
 {
   if (mode == MODE_COUNT)
-    AXB_LAUNCH((k_nlist<F, FULL, MODE_COUNT>), dim3(grid_of(nl)), dim3(256), 0, s, tv, radius,
+    AXB_LAUNCH((k_nlist<F, MODE_COUNT>), dim3(grid_of(nl)), dim3(256), 0, s, tv, radius,
                nl, list, offsets, out, buffer, rowof);
   else if (mode == MODE_FILL)
-    AXB_LAUNCH((k_nlist<F, FULL, MODE_FILL>), dim3(grid_of(nl)), dim3(256), 0, s, tv, radius,
+    AXB_LAUNCH((k_nlist<F, MODE_FILL>), dim3(grid_of(nl)), dim3(256), 0, s, tv, radius,
                nl, list, offsets, out, buffer, rowof);
   else
-    AXB_LAUNCH((k_nlist<F, FULL, MODE_BUFFER>), dim3(grid_of(nl)), dim3(256), 0, s, tv, radius,
+    AXB_LAUNCH((k_nlist<F, MODE_BUFFER>), dim3(grid_of(nl)), dim3(256), 0, s, tv, radius,
                nl, list, offsets, out, buffer, rowof);
   return hipGetLastError();
 }
@@ -2435,25 +2434,19 @@ static hipError_t launch_nlist_group(const TreeView &tv, float radius, int64_t n
 
 hipError_t launch_nlist(const TreeView &tv, int node_format, bool full, float radius, int64_t nl,
                         const uint32_t *list, int64_t *offsets, int32_t *out, int32_t buffer,
-                        uint32_t *rowof, int mode, bool group, hipStream_t s)
+                        uint32_t *rowof, int mode, hipStream_t s)
 {
   if (nl <= 0)
     return hipSuccess;
-  if (group && full && tv.leaves)
-    return node_format == NODES_Q16
-               ? launch_nlist_group<NODES_Q16>(tv, radius, nl, list, offsets, out, buffer, rowof,
-                                               mode, s)
-               : launch_nlist_group<NODES_FP32>(tv, radius, nl, list, offsets, out, buffer,
-                                                rowof, mode, s);
   if (node_format == NODES_Q16)
-    return full ? launch_nlist_f<NODES_Q16, true>(tv, radius, nl, list, offsets, out, buffer,
-                                                  rowof, mode, s)
-                : launch_nlist_f<NODES_Q16, false>(tv, radius, nl, list, offsets, out, buffer,
-                                                   rowof, mode, s);
-  return full ? launch_nlist_f<NODES_FP32, true>(tv, radius, nl, list, offsets, out, buffer,
-                                                 rowof, mode, s)
-              : launch_nlist_f<NODES_FP32, false>(tv, radius, nl, list, offsets, out, buffer,
-                                                  rowof, mode, s);
+    return full ? launch_nlist_group<NODES_Q16>(tv, radius, nl, list, offsets, out, buffer,
+                                                rowof, mode, s)
+                : launch_nlist_half<NODES_Q16>(tv, radius, nl, list, offsets, out, buffer, rowof,
+                                               mode, s);
+  return full ? launch_nlist_group<NODES_FP32>(tv, radius, nl, list, offsets, out, buffer, rowof,
+                                               mode, s)
+              : launch_nlist_half<NODES_FP32>(tv, radius, nl, list, offsets, out, buffer, rowof,
+                                              mode, s);
 }
 
 hipError_t launch_h2f_count(const int64_t *offsets, const int32_t *indices, int64_t n,
