@@ -66,3 +66,26 @@ def test_directions_with_tiny_components():
         i, o = tree.query(ax.ordered_intersects(r))
         np.testing.assert_array_equal(o.cpu().numpy(), o_ref)
         np.testing.assert_array_equal(i.cpu().numpy(), i_ref)
+
+
+@pytest.mark.parametrize("fmt", ["fp32", "q16"])
+@pytest.mark.parametrize("k", [1, 4, 8])
+def test_stack_past_its_entries(k, fmt):
+    # 19 scales times three axes, eight equal boxes each, split one after the
+    # other from the rest of the tree, and 65536 equal boxes at its end: the
+    # way down to them passes more than 64 nodes, all around the rays' origins
+    boxes = []
+    for i in range(1, 20):
+        for a in range(3):
+            c = np.zeros(3)
+            c[a] = 2.0 ** -i
+            boxes += [np.concatenate([c - 1.5 * 2.0 ** -i, c + 1.5 * 2.0 ** -i])] * 8
+    tip = 1.5 * 2.0 ** -20
+    boxes += [np.array([-tip] * 3 + [tip] * 3)] * 65536
+    boxes = np.array(boxes, np.float32)[np.random.default_rng(k).permutation(len(boxes))]
+    g = np.random.default_rng(1)
+    rays = oracle.make_rays(np.zeros((5, 3), np.float32), g.normal(size=(5, 3)).astype(np.float32))
+    with ax.profile(timing=True) as prof:
+        _check(boxes, rays, k, fmt)
+    # the rows were taken from the whole ordered ones instead
+    assert any("k_row_prefix_copy" in n for n in prof.kernels)
