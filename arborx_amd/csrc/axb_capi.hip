@@ -162,6 +162,9 @@ void pool_free(void *p, hipStream_t stream)
 // (beyond it the blocks freed longest ago go back to the pool, see dfree),
 // axb_trim_memory returns all of it, and an allocation that fails, of
 // whatever kind, empties the lists before it gives up (pool_alloc).
+// A destroyed stream's handle may be given to a new stream, which then finds
+// the old one's blocks: hipStreamDestroy returns when the stream's work is
+// done (4.25 ms behind a kernel of 4.3), so they are idle by then.
 // hipStreamPerThread is one handle for a stream per thread, so its blocks
 // bypass the cache.
 namespace

@@ -107,8 +107,8 @@ AXB_D WalkCost rope_walk_cost(const TreeView &tv, const int64_t *__restrict__ of
 }
 
 // Spheres against points, 64 lanes searching together (axb_group.hpp).  10M
-// uniform points, ~32 neighbours: 5.31 (k_spatial) -> 2.27 ms, 6650 vector
-// instructions per wavefront, 72% of the issue rate; six wavefronts per SIMD
+// uniform points, ~32 neighbours: 5.31 (k_spatial) -> 2.31 ms, 6720 vector
+// instructions per wavefront, 74% of the issue rate; six wavefronts per SIMD
 // (80 registers, 25 KB of LDS per block; four with windows of 8 words: 2.44).
 // Hits leave in groups of four: a row's hits follow closely here, so its
 // 16-byte stores meet in L2 (through an LDS stage of 16 per lane: 3.4 ms, the
@@ -1453,7 +1453,7 @@ AXB_D float group_row_bound(const uint2 *__restrict__ cand, uint32_t row_at, int
 // (limit), search alone as in k_knn_collect.  EVEN: the radius is guessed
 // from the group's density (spacing: of the leaves), else from each lane's
 // own (spacing: leaves per query).  10M uniform points, k = 16: 9.14
-// (k_knn_collect) -> 4.25 ms, 13300 vector instructions per wavefront, 79%
+// (k_knn_collect) -> 4.35 ms, 13300 vector instructions per wavefront, 78%
 // of the issue rate: about half the exact tests of the ~38 leaves a lane
 // finds, a fifth the selection; five wavefronts per SIMD (six: 4.36 ms, 26
 // registers spilled).  The limit costs 0.14 ms there, so batches over uniform

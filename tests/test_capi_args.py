@@ -159,3 +159,12 @@ def test_debug_limits_arguments():
     assert L.axb_debug_set_limits(0, 0, 65) == INVALID
     assert L.axb_debug_set_limits(0, 0, -2) == INVALID
     assert L.axb_debug_set_limits(0, 0, 0) == ax.AXB_OK
+
+
+def test_debug_memory_and_search_arguments():
+    L = ax.lib()
+    assert L.axb_debug_set_memory(0, -1) == INVALID
+    assert L.axb_debug_set_memory(0, 0) == ax.AXB_OK
+    for knn_small, fill in ((-1, 0), (0, -2), (0, 4)):
+        assert L.axb_debug_set_search(knn_small, fill) == INVALID
+    assert L.axb_debug_set_search(0, -1) == ax.AXB_OK
