@@ -2000,12 +2000,14 @@ int knn_row_capacity(int k, int n) { return knn_shape(k, n).cap; }
 // Leaves the group search aims at for k nearest: a count that is Poisson
 // around k + 4 sqrt(k) + 4 falls below k once in ~10^4.
 static float knn_group_want(int k) { return (float)k + 4.f * std::sqrt((float)k) + 4.f; }
-// Up to this many queries a launch is as long as its slowest wavefronts.
-static int64_t knn_small()
+// From this many queries on few neighbours pay in groups over uneven leaves.
+static int64_t knn_many()
 {
-  const int64_t lim = debug_limits().knn_small;
-  return lim > 0 ? lim : 300000;
+  const int64_t lim = debug_limits().knn_many;
+  return lim > 0 ? lim : 1000000;
 }
+// Up to this many queries a launch is as long as its slowest wavefronts.
+constexpr int64_t KNN_SMALL = 300000;
 // The most candidates a group may search: what they cost (group_cost) is then
 // that of 64 lanes' own walks, about 8800 + 1360 vector instructions per leaf
 // wanted.
@@ -2020,22 +2022,28 @@ static LeafLimit knn_leaf_limit(int k)
 // ones sees too many leaves: 1M clustered points, 130k queries, k = 10 0.61
 // -> 0.83 ms), for k >= 2 (the nearest one of 4M uniform points: 0.90 ms
 // alone, 1.03 in groups), and where the leaves fill space evenly enough for
-// the guessed radius to be right (TreeView::fill).  Calls, alone / in groups
-// of k_knn_collect_group<.., NoLimit>, in ms:
-//   even         1M uniform, k = 10           1.02 / 0.65
-//                250k normal, k = 10          0.72 / 0.71
-//   uneven       1M on a sphere, k = 10       1.06 / 1.23, k = 24 2.12 / 1.62
-//                1M in 1000 clusters, k = 10  1.49 / 1.52, k = 24 3.21 / 2.42
-//                50k on a sphere, k = 5       0.35 / 0.35, k = 10 0.44 / 0.44
-//                  (with the limit                   0.29              0.31)
-//   thin         1M on a line, k = 24         2.04 / 4.99
-//                50k in 20 clusters, k = 10   0.68 / 1.94, k = 24 1.55 / 2.70
+// the guessed radius to be right (TreeView::fill).  Calls in ms, alone / in
+// groups (thin: without a limit):
+//   even    1M uniform, k = 10      1.02 / 0.65
+//           250k normal, k = 10     0.72 / 0.71
+//   thin    1M on a line, k = 24    2.04 / 4.99
+//           50k in 20 clusters, k = 10  0.68 / 1.94, k = 24 1.55 / 2.70
+//   uneven             on a sphere                 in 1000 clusters
+//           k = 2          5          10           2          5         10
+//    100k                         0.42/0.38                         0.49/0.35
+//    300k  .38/.48    .44/.54    .57/.60       .42/.43    .64/.65    .79/.78
+//    600k  .50/.45    .61/.58    .75/.82       .60/.60    .87/.79   1.09/1.16
+//    1M    .61/.72    .77/.79   1.06/0.93      .75/.77   1.09/1.01  1.57/1.39
+//    4M   1.75/1.62  2.31/2.07  3.20/2.72     2.15/1.87  3.12/2.46  4.49/3.45
+//    10M  4.11/3.56  5.51/4.52  8.04/5.93     4.88/4.06  7.11/5.25 10.47/6.97
+// Of 12 sets, a tenth as wide clusters among them, k = 2 is up to a fifth
+// slower in groups at 1M and 10M, and k = 5 no more than 5% from 1M on.
 bool knn_group_rule(const TreeView &tv, int64_t nq, int k)
 {
   return tv.leaves && k >= 2 && k <= 64 && nq * 2 >= tv.n &&
          (float)tv.n >= 8.f * knn_group_want(k) &&
          (tv.fill >= FILL_EVEN ||
-          (tv.fill == FILL_UNEVEN && (k >= 20 || (k >= 8 && nq <= knn_small()))));
+          (tv.fill == FILL_UNEVEN && (k >= 8 || (k >= 5 && nq >= knn_many()))));
 }
 
 template <int F, int G, int K>
@@ -2059,7 +2067,7 @@ static hipError_t knn_run(const TreeView &tv, const float *pts, int64_t nq, int 
   // small launches over uniform leaves guess from the group's density: fewer
   // groups need a second round (calls of 250k points, k = 10: 0.28 ms, 0.34
   // from the lanes' own; normal ones, k = 5, 0.55 / 0.48)
-  const bool small = nq <= knn_small();
+  const bool small = nq <= KNN_SMALL;
   for (int64_t t0 = 0; e == hipSuccess && t0 < nq; t0 += ws.batch)
   {
     const int64_t tn = std::min(ws.batch, nq - t0);

@@ -252,11 +252,23 @@ def test_nearest_in_groups_where_leaves_fill_space(k, grouped):
         _check_nearest(p, p, k)
 
 
+@pytest.mark.parametrize("k,n,group", [(4, 1000000, False), (5, 999999, False),
+                                       (5, 1000000, True), (8, 400000, True),
+                                       (16, 400000, True)])
+def test_nearest_of_many_uneven_queries_in_groups(k, n, group):
+    g = np.random.default_rng(6)
+    p = g.uniform(size=(1000, 3))[np.arange(n) % 1000] + 0.01 * g.normal(size=(n, 3))
+    p = p.astype(np.float32)
+    kernels = _knn_kernels(p, k)
+    assert ["k_knn_collect_group" in name for name in kernels] == [group]
+    _check_nearest(p, p, k)
+
+
 @pytest.mark.parametrize("fill", [0, 1, 2, 3])
 @pytest.mark.parametrize("k", [2, 3, 5, 8, 13, 16, 17, 24, 32, 33, 64])
 def test_nearest_over_every_route(k, fill):
     # uneven density, duplicates, ties and queries without an answer, through
-    # each guess of the radius and as small and as large launches
+    # each guess of the radius, as few and as many queries
     g = np.random.default_rng(k)
     p = g.uniform(size=(7000, 3))
     p[:3000] = g.uniform(size=(30, 3))[np.arange(3000) % 30]
@@ -276,9 +288,9 @@ def test_nearest_over_every_route(k, fill):
         ax.make_nearest(torch.from_numpy(bad), k))[0].reshape(-1, k)
     keep = torch.from_numpy(np.isfinite(bad).all(1)).cuda()
     tree = ax.BVH(torch.from_numpy(p).cuda(), node_format="fp32" if k % 2 else "q16")
-    for small in (1, 1 << 30):
+    for many in (1, 1 << 30):
         for limits in (dict(), dict(knn_batch_max=777)):
-            with ax.debug_search(knn_small=small, fill=fill), ax.debug_limits(**limits):
+            with ax.debug_search(knn_many=many, fill=fill), ax.debug_limits(**limits):
                 i, o, d = tree.query(ax.make_nearest(torch.from_numpy(q), k),
                                      return_distances=True)
                 b = tree.query(ax.make_nearest(torch.from_numpy(bad), k))[0].reshape(-1, k)
