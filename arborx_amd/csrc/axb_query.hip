@@ -1458,11 +1458,22 @@ AXB_D float group_row_bound(const uint2 *__restrict__ cand, uint32_t row_at, int
 // finds, a fifth the selection; five wavefronts per SIMD (six: 4.36 ms, 26
 // registers spilled).  The limit costs 0.14 ms there, so batches over uniform
 // leaves, where every group pays, go without.
+// Lanes farther than a margin outside the points walk alone from the start:
+// the density around them says nothing of their radius, and the lanes of an
+// outside group are far apart (200k uniform points, as many queries in a cube
+// of 1.5 times the side, k = 16: 2.34 -> 0.80 ms; 4M 10.92 / 10.98).
 constexpr int GROUP_ROUNDS = 6;
+AXB_D float scene_d2(const Box6 &b, float x, float y, float z)
+{
+  const float dx = fmaxf(fmaxf(b.lo[0] - x, x - b.hi[0]), 0.f);
+  const float dy = fmaxf(fmaxf(b.lo[1] - y, y - b.hi[1]), 0.f);
+  const float dz = fmaxf(fmaxf(b.lo[2] - z, z - b.hi[2]), 0.f);
+  return dx * dx + dy * dy + dz * dz;
+}
 template <int F, int K, bool EVEN, class Limit>
 __global__ __launch_bounds__(256, K <= 16 ? 5 : (K <= 32 ? 4 : 2)) void k_knn_collect_group(
     TreeView tv, const float *__restrict__ pts, int64_t t0, int64_t tn, int k, float want,
-    float spacing, Limit limit, int W, float shrink, const uint32_t *__restrict__ order,
+    float spacing, float margin, Limit limit, int W, float shrink, const uint32_t *__restrict__ order,
     uint2 *__restrict__ cand, int cap, int max_rounds, uint32_t *__restrict__ ovf, uint32_t *__restrict__ ovf_n,
     int32_t *__restrict__ oi, float *__restrict__ od)
 {
@@ -1479,7 +1490,8 @@ __global__ __launch_bounds__(256, K <= 16 ? 5 : (K <= 32 ? 4 : 2)) void k_knn_co
   }
   const int m = k < tv.n ? k : tv.n;
   GroupLds &L = s_group[threadIdx.x >> 6];
-  bool pending = real && fabsf(x) < INFINITY && fabsf(y) < INFINITY && fabsf(z) < INFINITY;
+  bool pending = real && fabsf(x) < INFINITY && fabsf(y) < INFINITY && fabsf(z) < INFINITY &&
+                 scene_d2(tv.scene, x, y, z) <= margin * margin;
   uint32_t v_int = 0, v_leaf = 0;
   GroupCand row{cand, real ? (uint32_t)(g * cap) : 0u, cap, 0, make_uint2(0u, 0u)};
   int c = 0, rounds = 0;
@@ -2064,6 +2076,8 @@ static hipError_t knn_run(const TreeView &tv, const float *pts, int64_t nq, int 
     vol *= std::max(tv.scene.hi[d] - tv.scene.lo[d], 1e-3f * longest);
   const float spacing = std::cbrt(vol / (float)tv.n);
   const float per_query = (float)tv.n / (float)nq;
+  // the ball that holds the target at the tree's mean density
+  const float margin = std::cbrt(0.2387f * want) * spacing;
   // small launches over uniform leaves guess from the group's density: fewer
   // groups need a second round (calls of 250k points, k = 10: 0.28 ms, 0.34
   // from the lanes' own; normal ones, k = 5, 0.55 / 0.48)
@@ -2077,15 +2091,15 @@ static hipError_t knn_run(const TreeView &tv, const float *pts, int64_t nq, int 
       group = order && knn_group_rule(tv, nq, k);
       if (group && tv.fill == FILL_UNIFORM && small)
         AXB_LAUNCH((k_knn_collect_group<F, K, true, NoLimit>), dim3(grid_of(tn)), dim3(256), 0, s,
-                   tv, pts, t0, tn, k, want, spacing, NoLimit{}, sh.W, sh.shrink, order, ws.cand,
+                   tv, pts, t0, tn, k, want, spacing, margin, NoLimit{}, sh.W, sh.shrink, order, ws.cand,
                    sh.cap, rounds, ws.ovf, ws.ovf_n, oi, od);
       else if (group && tv.fill == FILL_UNIFORM)
         AXB_LAUNCH((k_knn_collect_group<F, K, false, NoLimit>), dim3(grid_of(tn)), dim3(256), 0, s,
-                   tv, pts, t0, tn, k, want, per_query, NoLimit{}, sh.W, sh.shrink, order, ws.cand,
+                   tv, pts, t0, tn, k, want, per_query, margin, NoLimit{}, sh.W, sh.shrink, order, ws.cand,
                    sh.cap, rounds, ws.ovf, ws.ovf_n, oi, od);
       else if (group)
         AXB_LAUNCH((k_knn_collect_group<F, K, false, LeafLimit>), dim3(grid_of(tn)), dim3(256), 0,
-                   s, tv, pts, t0, tn, k, want, per_query, knn_leaf_limit(k), sh.W, sh.shrink,
+                   s, tv, pts, t0, tn, k, want, per_query, margin, knn_leaf_limit(k), sh.W, sh.shrink,
                    order, ws.cand, sh.cap, rounds, ws.ovf, ws.ovf_n, oi, od);
     }
     if (group)

@@ -252,6 +252,19 @@ def test_nearest_in_groups_where_leaves_fill_space(k, grouped):
         _check_nearest(p, p, k)
 
 
+def test_nearest_of_queries_outside_the_points():
+    # far outside, the leaves' density is no guide to a radius: such lanes
+    # walk alone (135 records per query, 270 where they search as a group)
+    n = 200000
+    p = synthetic.uniform_points(n, 1)
+    q = synthetic.uniform_points(n, 2) * np.float32(1.5) - np.float32(0.25)
+    tree = ax.BVH(torch.from_numpy(p).cuda(), node_format="q16")
+    with ax.profile(timing=False, visits=True) as prof:
+        tree.query(ax.make_nearest(torch.from_numpy(q), 5))
+    assert prof.visits["leaf"] < 200 * n
+    _check_nearest(p, q, 5)
+
+
 @pytest.mark.parametrize("k,n,group", [(4, 1000000, False), (5, 999999, False),
                                        (5, 1000000, True), (8, 400000, True),
                                        (16, 400000, True)])
