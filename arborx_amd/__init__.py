@@ -715,16 +715,16 @@ class debug_limits:
 
 class debug_search:
     """Replaces what the rules of the searches of 64 lanes together go by
-    (tests only; process-wide): the nearest queries from which few neighbours
-    in uneven sets are searched together and how the leaves fill space (0
-    thinly .. 3 uniformly, -1: as measured).
+    (tests only; process-wide): the nearest queries from which a launch counts
+    as large and how the leaves fill space (0 thinly .. 3 uniformly, -1: as
+    measured).
 
-    with arborx_amd.debug_search(knn_many=1, fill=2):
+    with arborx_amd.debug_search(knn_large=1, fill=2):
         ...
     """
 
-    def __init__(self, knn_many=0, fill=-1):
-        self.args = (int(knn_many), int(fill))
+    def __init__(self, knn_large=0, fill=-1):
+        self.args = (int(knn_large), int(fill))
 
     def __enter__(self):
         _check(lib().axb_debug_set_search(*self.args))

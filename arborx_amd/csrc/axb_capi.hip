@@ -444,14 +444,14 @@ std::map<WsKey, std::array<WsBlock, WS_NUM>> g_ws;
 std::atomic<int64_t> g_lim_knn_batch{0};
 std::atomic<int64_t> g_lim_rows_bytes{0};
 std::atomic<int32_t> g_lim_knn_rounds{0};
-std::atomic<int64_t> g_lim_knn_many{0};
+std::atomic<int64_t> g_lim_knn_large{0};
 std::atomic<int32_t> g_lim_fill{0};
 } // namespace
 
 Limits debug_limits()
 {
   return Limits{g_lim_knn_batch.load(), g_lim_rows_bytes.load(), g_lim_knn_rounds.load(),
-                g_lim_knn_many.load(), g_lim_fill.load()};
+                g_lim_knn_large.load(), g_lim_fill.load()};
 }
 
 void WsLease::acquire(hipStream_t s_, int slot_, size_t bytes)
@@ -729,11 +729,11 @@ axb_status axb_debug_set_limits(int64_t knn_batch_max, int64_t scratch_rows_byte
   return AXB_OK;
 }
 
-axb_status axb_debug_set_search(int64_t knn_many, int32_t fill)
+axb_status axb_debug_set_search(int64_t knn_large, int32_t fill)
 {
-  if (knn_many < 0 || fill < -1 || fill > FILL_UNIFORM)
+  if (knn_large < 0 || fill < -1 || fill > FILL_UNIFORM)
     AXB_FAIL(AXB_ERR_INVALID_ARGUMENT, "axb_debug_set_search: bad limit");
-  g_lim_knn_many.store(knn_many);
+  g_lim_knn_large.store(knn_large);
   g_lim_fill.store(fill + 1);
   return AXB_OK;
 }

@@ -105,7 +105,7 @@ struct Limits
   int64_t knn_batch_max;      // kNN queries per collect launch
   int64_t scratch_rows_bytes; // scratch rows of a buffered CRS query
   int32_t knn_rounds;         // collect rounds before the exact fallback
-  int64_t knn_many;           // kNN queries from which few neighbours pay in groups
+  int64_t knn_large;          // kNN queries of a large launch
   int32_t fill;               // 1 + FILL_*
 };
 Limits debug_limits();

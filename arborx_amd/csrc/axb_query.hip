@@ -2012,14 +2012,14 @@ int knn_row_capacity(int k, int n) { return knn_shape(k, n).cap; }
 // Leaves the group search aims at for k nearest: a count that is Poisson
 // around k + 4 sqrt(k) + 4 falls below k once in ~10^4.
 static float knn_group_want(int k) { return (float)k + 4.f * std::sqrt((float)k) + 4.f; }
-// From this many queries on few neighbours pay in groups over uneven leaves.
-static int64_t knn_many()
+// Whether a launch counts as large (the debug limit moves every such line).
+constexpr int64_t KNN_LARGE_UNIFORM = 300000; // see knn_run
+constexpr int64_t KNN_LARGE_UNEVEN = 1000000; // see knn_group_rule
+static bool knn_large(int64_t nq, int64_t line)
 {
-  const int64_t lim = debug_limits().knn_many;
-  return lim > 0 ? lim : 1000000;
+  const int64_t lim = debug_limits().knn_large;
+  return nq >= (lim > 0 ? lim : line);
 }
-// Up to this many queries a launch is as long as its slowest wavefronts.
-constexpr int64_t KNN_SMALL = 300000;
 // The most candidates a group may search: what they cost (group_cost) is then
 // that of 64 lanes' own walks, about 8800 + 1360 vector instructions per leaf
 // wanted.
@@ -2055,7 +2055,7 @@ bool knn_group_rule(const TreeView &tv, int64_t nq, int k)
   return tv.leaves && k >= 2 && k <= 64 && nq * 2 >= tv.n &&
          (float)tv.n >= 8.f * knn_group_want(k) &&
          (tv.fill >= FILL_EVEN ||
-          (tv.fill == FILL_UNEVEN && (k >= 8 || (k >= 5 && nq >= knn_many()))));
+          (tv.fill == FILL_UNEVEN && (k >= 8 || (k >= 5 && knn_large(nq, KNN_LARGE_UNEVEN)))));
 }
 
 template <int F, int G, int K>
@@ -2078,10 +2078,14 @@ static hipError_t knn_run(const TreeView &tv, const float *pts, int64_t nq, int 
   const float per_query = (float)tv.n / (float)nq;
   // the ball that holds the target at the tree's mean density
   const float margin = std::cbrt(0.2387f * want) * spacing;
-  // small launches over uniform leaves guess from the group's density: fewer
-  // groups need a second round (calls of 250k points, k = 10: 0.28 ms, 0.34
-  // from the lanes' own; normal ones, k = 5, 0.55 / 0.48)
-  const bool small = nq <= KNN_SMALL;
+  // Below the line over uniform leaves the radius comes from the group's
+  // density, from it on from each lane's own.  Uniform points hardly ask
+  // for the line (own / group's, calls in ms, k = 10: 300k 0.33 / 0.29, 600k
+  // 0.49 / 0.44, 1M 0.63 / 0.60, 4M 1.88 / 1.85, 10M 4.29 / 4.29), uneven
+  // spots among them do (a twentieth of the points in a clump: 400k 0.52 /
+  // 0.59, 1M 0.68 / 0.76, 4M 1.91 / 1.91), and so do uneven leaves (250k
+  // normal points, k = 5 0.48 / 0.55).
+  const bool small = !knn_large(nq, KNN_LARGE_UNIFORM);
   for (int64_t t0 = 0; e == hipSuccess && t0 < nq; t0 += ws.batch)
   {
     const int64_t tn = std::min(ws.batch, nq - t0);

@@ -443,13 +443,13 @@ axb_status axb_debug_set_limits(int64_t knn_batch_max, int64_t scratch_rows_byte
                                 int32_t knn_rounds);
 
 /* Test hook for the rules of the searches of 64 lanes together (no reference
- * counterpart): knn_many replaces the number of nearest queries from which few
- * neighbours in uneven sets are searched together (0: the default); fill how
- * a point tree's leaves are taken to fill space, 0 thinly (surfaces, curves,
+ * counterpart): knn_large replaces the number of nearest queries from which a
+ * launch counts as large (0: the defaults, which differ by rule); fill how a
+ * point tree's leaves are taken to fill space, 0 thinly (surfaces, curves,
  * tight clusters), 1 unevenly, 2 evenly, 3 uniformly (-1: as measured when it
  * was built).
  * Process-wide; set it between calls. */
-axb_status axb_debug_set_search(int64_t knn_many, int32_t fill);
+axb_status axb_debug_set_search(int64_t knn_large, int32_t fill);
 
 /* Test hooks for the device blocks kept between calls (no reference
  * counterpart): scarce != 0 makes every allocation fail while blocks are

@@ -165,6 +165,6 @@ def test_debug_memory_and_search_arguments():
     L = ax.lib()
     assert L.axb_debug_set_memory(0, -1) == INVALID
     assert L.axb_debug_set_memory(0, 0) == ax.AXB_OK
-    for knn_many, fill in ((-1, 0), (0, -2), (0, 4)):
-        assert L.axb_debug_set_search(knn_many, fill) == INVALID
+    for knn_large, fill in ((-1, 0), (0, -2), (0, 4)):
+        assert L.axb_debug_set_search(knn_large, fill) == INVALID
     assert L.axb_debug_set_search(0, -1) == ax.AXB_OK

@@ -281,7 +281,7 @@ def test_nearest_of_many_uneven_queries_in_groups(k, n, group):
 @pytest.mark.parametrize("k", [2, 3, 5, 8, 13, 16, 17, 24, 32, 33, 64])
 def test_nearest_over_every_route(k, fill):
     # uneven density, duplicates, ties and queries without an answer, through
-    # each guess of the radius, as few and as many queries
+    # each guess of the radius and as small and as large launches
     g = np.random.default_rng(k)
     p = g.uniform(size=(7000, 3))
     p[:3000] = g.uniform(size=(30, 3))[np.arange(3000) % 30]
@@ -301,9 +301,9 @@ def test_nearest_over_every_route(k, fill):
         ax.make_nearest(torch.from_numpy(bad), k))[0].reshape(-1, k)
     keep = torch.from_numpy(np.isfinite(bad).all(1)).cuda()
     tree = ax.BVH(torch.from_numpy(p).cuda(), node_format="fp32" if k % 2 else "q16")
-    for many in (1, 1 << 30):
+    for large in (1, 1 << 30):
         for limits in (dict(), dict(knn_batch_max=777)):
-            with ax.debug_search(knn_many=many, fill=fill), ax.debug_limits(**limits):
+            with ax.debug_search(knn_large=large, fill=fill), ax.debug_limits(**limits):
                 i, o, d = tree.query(ax.make_nearest(torch.from_numpy(q), k),
                                      return_distances=True)
                 b = tree.query(ax.make_nearest(torch.from_numpy(bad), k))[0].reshape(-1, k)
