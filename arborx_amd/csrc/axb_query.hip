@@ -108,8 +108,9 @@ AXB_D WalkCost rope_walk_cost(const TreeView &tv, const int64_t *__restrict__ of
 
 // Spheres against points, 64 lanes searching together (axb_group.hpp).  10M
 // uniform points, ~32 neighbours: 5.31 (k_spatial) -> 2.31 ms, 6720 vector
-// instructions per wavefront, 74% of the issue rate; six wavefronts per SIMD
-// (80 registers, 25 KB of LDS per block; four with windows of 8 words: 2.44).
+// instructions per wavefront, 74% of the issue rate (2.13 ms and 80% on a
+// faster card); six wavefronts per SIMD (80 registers, 25 KB of LDS per block;
+// four with windows of 8 words: 2.44).
 // Hits leave in groups of four: a row's hits follow closely here, so its
 // 16-byte stores meet in L2 (through an LDS stage of 16 per lane: 3.4 ms, the
 // stage's LDS cost a third of the wavefronts).
@@ -1454,10 +1455,10 @@ AXB_D float group_row_bound(const uint2 *__restrict__ cand, uint32_t row_at, int
 // from the group's density (spacing: of the leaves), else from each lane's
 // own (spacing: leaves per query).  10M uniform points, k = 16: 9.14
 // (k_knn_collect) -> 4.35 ms, 13300 vector instructions per wavefront, 78%
-// of the issue rate: about half the exact tests of the ~38 leaves a lane
-// finds, a fifth the selection; five wavefronts per SIMD (six: 4.36 ms, 26
-// registers spilled).  The limit costs 0.14 ms there, so batches over uniform
-// leaves, where every group pays, go without.
+// of the issue rate (4.26 ms and 80% on a faster card): about half the exact
+// tests of the ~38 leaves a lane finds, a fifth the selection; five wavefronts
+// per SIMD (six: 4.36 ms, 26 registers spilled).  The limit costs 0.14 ms
+// there, so batches over uniform leaves, where every group pays, go without.
 // Lanes farther than a margin outside the points walk alone from the start:
 // the density around them says nothing of their radius, and the lanes of an
 // outside group are far apart (200k uniform points, as many queries in a cube
